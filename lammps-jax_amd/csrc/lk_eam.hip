@@ -2,8 +2,8 @@
 // the one-sided full-list scheme of python/lammps_jax/eam_pallas.py:181-249).
 //
 // Both sweeps walk the row tiles written by the pack (lk_pack.hip, lk_tile.h): one lane per list
-// row, the waves of a tile advancing the kept-entry ordinal k together, so the receivers of one
-// step are read as one contiguous run. A row's sums stay in registers and meet across waves in
+// row, each wave of a tile taking its share of the kept-entry ordinals (OwnEdges), so the receivers
+// of one step are read as one contiguous run. A row's sums stay in registers and meet across waves in
 // LDS in a fixed order: no float atomics, bitwise reproducible runs.
 //
 // Spline tables live in LDS. Each (node, table) entry is 16 bytes: in float64 the node's value
@@ -27,9 +27,33 @@
 namespace lk {
 
 constexpr int kDensW = 4, kDensTPB = 4, kDensLds = 4096;     // 64 KB table window
-// two waves per 64-row tile, eight tiles per block (C3 force rows: 4 x 4 took 77.6 us, 2 x 8
-// 73 us, 8 x 2 91.5 us, 1 x 16 113.5 us)
-constexpr int kForceW = 2, kForceTPB = 8, kForceLds = 7680;  // 120 KB table window
+constexpr int kForceWaves = 16, kForceLds = 7680;  // waves per force block, 120 KB table window
+
+// Waves per 64-row tile of the force sweep; a block's sixteen waves hold 16 / W tiles. One block
+// fits a CU (the table window), so a sweep takes as many rounds as its tiles fill CUs at 16 / W
+// tiles apiece, and a round's time falls with W less than in proportion (the window fill, the
+// rows' loads and the sums stay): t ~ rounds * (1 / W + 0.06), fitted to the times below. Two
+// waves per tile at every size left most CUs idle under 2,048 tiles: force sweep in us, float64,
+// by W = 2, 4, 8, 16 (the rule's choice starred):
+//   14 tiles (840 atoms) 57, 35, 24, 19*    1,024 tiles (65,536) 59, 38*, 44, 54
+//   128 tiles (8,192)    57, 35, 25, 21*    1,630 tiles (104,284) 61*, 62, 71, 82
+//   465 tiles (29,716)   59, 36, 27*, 33    2,048 tiles (131,072) 62*, 63, 74, 93
+//   2,112 tiles (135,168) 103, 84, 84*, 102    3,600 tiles (230,400) 110*, 113, 126, 161
+static int force_waves_per_tile(int ntiles, int num_cus)
+{
+  const int cus = num_cus > 0 ? num_cus : 256;
+  int best = 2;
+  double least = 0.0;
+  for (int w = 2; w <= kForceWaves; w *= 2) {
+    const int per_round = cus * (kForceWaves / w);
+    const double t = ((ntiles + per_round - 1) / per_round) * (1.0 / w + 0.06);
+    if (w == 2 || t < least) {
+      best = w;
+      least = t;
+    }
+  }
+  return best;
+}
 
 // Density sweep (one-sided): rho_i over the row's own edges, then F(rho_i), F'(rho_i). Owned rows
 // add F(rho_i) to the tile's energy partial.
@@ -50,7 +74,7 @@ __global__ __launch_bounds__(W * TPB * 64) LK_EIGHT_WAVES void k_eam_density_row
     const int cnt = i >= 0 ? a.row_count[ii] : 0;
     Atom4<S> ai = {S(0), S(0), S(0), S(0)};
     if (i >= 0) ai = a.atoms[i];
-    const long base = tile * kWave < a.num_rows ? a.tile_off[tile] : 0;
+    const int base = tile * kWave < a.num_rows ? a.tile_off[tile] : 0;
     S rho = S(0);
     struct Rec {
       Atom4<S> at;
@@ -192,7 +216,7 @@ __global__ __launch_bounds__(W * TPB * 64) void k_eam_force_rows(EamArgs<S> a, i
   // records and F'; and each tile's embedding energy (slot 0 of its partials, from an earlier
   // launch), held by thread q < TPB for tile q until the group's sums.
   int i = -1, cnt = 0;
-  long base = 0;
+  int base = 0;
   double emb = 0.0;
   auto load_ids = [&](int g) {
     const int tile = g * TPB + sub;
@@ -431,22 +455,33 @@ static hipError_t eam_onesided(Handle &h, hipStream_t s, int nlocal, int nghost,
   return launch_eam_force(h, s, a, flags);
 }
 
-template <typename S>
-hipError_t launch_eam_force_t(Handle &h, hipStream_t s, EamArgs<S> a, int flags)
+template <typename S, int W>
+static hipError_t launch_eam_force_w(Handle &h, hipStream_t s, const EamArgs<S> &a)
 {
+  constexpr int TPB = kForceWaves / W;
   // One launch even with no rows: its last block writes the step result.
-  const int ntiles = a.ntiles;
-  const int ngroups = ntiles > 0 ? (ntiles + kForceTPB - 1) / kForceTPB : 1;
+  const int ngroups = a.ntiles > 0 ? (a.ntiles + TPB - 1) / TPB : 1;
   const int grid = persistent_grid(ngroups, 1, h.num_cus);
-  a.flags = flags;
   StageTimer timer(h, s, "eam_force");
-  if (flags & LK_VIRIAL)
-    hipLaunchKernelGGL((k_eam_force_rows<S, kForceW, kForceTPB, true>), dim3(grid),
-                       dim3(kForceW * kForceTPB * kWave), 0, s, a, ngroups);
+  if (a.flags & LK_VIRIAL)
+    hipLaunchKernelGGL((k_eam_force_rows<S, W, TPB, true>), dim3(grid), dim3(kForceWaves * kWave),
+                       0, s, a, ngroups);
   else
-    hipLaunchKernelGGL((k_eam_force_rows<S, kForceW, kForceTPB, false>), dim3(grid),
-                       dim3(kForceW * kForceTPB * kWave), 0, s, a, ngroups);
+    hipLaunchKernelGGL((k_eam_force_rows<S, W, TPB, false>), dim3(grid), dim3(kForceWaves * kWave),
+                       0, s, a, ngroups);
   return hipGetLastError();
+}
+
+template <typename S>
+static hipError_t launch_eam_force_t(Handle &h, hipStream_t s, EamArgs<S> a, int flags)
+{
+  a.flags = flags;
+  switch (force_waves_per_tile(a.ntiles, h.num_cus)) {
+    case 16: return launch_eam_force_w<S, 16>(h, s, a);
+    case 8: return launch_eam_force_w<S, 8>(h, s, a);
+    case 4: return launch_eam_force_w<S, 4>(h, s, a);
+    default: return launch_eam_force_w<S, 2>(h, s, a);
+  }
 }
 
 hipError_t launch_eam_force(Handle &h, hipStream_t s, EamArgs<double> a, int flags)
