@@ -57,12 +57,11 @@ void free_all(Handle &h)
                   h.d_tile_off,  h.d_bits,      h.d_fp,          h.d_rho,       h.d_partials,
                   h.d_result,    h.d_ghost_owner, h.d_ghost_off, h.d_ghost_list, h.d_done,
                   h.d_deg,       h.d_inc_loc,   h.d_inc_part,    h.d_inc_tmp,   h.d_inc,
-                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_inc_bit,   h.d_edge_f,
+                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,
                   h.d_matrix,    h.d_num_neighbors, h.d_identity, h.d_inc_len,
                   h.tl.keys,     h.tl.keys_sorted, h.tl.rows_in, h.tl.order,  h.tl.sort_tmp,
                   h.tl.atom,     h.tl.nn,       h.tl.uni,        h.tl.ucount,   h.tl.lid,
-                  h.tl.box,      h.d_sort_keys, h.d_sort_vals,   h.d_sort_tmp,  h.d_sort_rows,
-                  h.d_sort_pre,  h.d_rowmark,   h.d_nonrow,      h.d_htab,      h.tl.ustat, h.d_dtab};
+                  h.tl.box,      h.d_row_of,    h.d_rowmark,   h.d_nonrow,      h.d_htab,      h.tl.ustat, h.d_dtab};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (h.h_result) (void)hipHostFree(h.h_result);
@@ -127,6 +126,7 @@ int ensure_incidence(Handle &h, long entries = 0)
     if ((e = dalloc(&h.d_inc_loc, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence offsets)");
     if ((e = dalloc(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
     if ((e = dalloc(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
+    if ((e = dalloc(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");
     if ((e = hipMalloc(&h.d_rho_part, A * h.scalar_bytes())) != hipSuccess) return hip_fail(h, e, "hipMalloc(rho partials)");
     if ((e = hipMalloc(&h.d_epair, A * h.scalar_bytes())) != hipSuccess) return hip_fail(h, e, "hipMalloc(pair energy)");
     if ((e = hipMemset(h.d_deg, 0, sizeof(int) * (A + 2))) != hipSuccess) return hip_fail(h, e, "hipMemset(incidence counts)");
@@ -143,16 +143,13 @@ int ensure_incidence(Handle &h, long entries = 0)
                 "fit in int)");
   if (need > h.inc_cap) {
     if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(h, e, "hipDeviceSynchronize");
-    for (void *p : {static_cast<void *>(h.d_inc_tmp), static_cast<void *>(h.d_inc),
-                    static_cast<void *>(h.d_inc_bit)})
+    for (void *p : {static_cast<void *>(h.d_inc_tmp), static_cast<void *>(h.d_inc)})
       if (p) (void)hipFree(p);
     h.d_inc_tmp = nullptr;
     h.d_inc = nullptr;
-    h.d_inc_bit = nullptr;
     h.inc_cap = 0;
     if ((e = dalloc(&h.d_inc_tmp, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence staging)");
     if ((e = dalloc(&h.d_inc, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lists)");
-    if ((e = dalloc(&h.d_inc_bit, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bits)");
     h.inc_cap = need;
     h.inc_key = Handle::IncKey{};  // rebuild
     fresh = true;

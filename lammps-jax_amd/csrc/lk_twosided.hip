@@ -28,20 +28,9 @@
 #include <cmath>
 #include <limits>
 
-#include <hipcub/hipcub.hpp>
-#include <rocprim/device/device_radix_sort.hpp>
-
 #include "lk_eam_common.h"
 
 namespace lk {
-
-// The in-entry sort of list-built lists: onesweep passes of 11-bit digits, so atom keys of up to
-// 22 bits (4 M atoms) take two passes over the pairs instead of three 8-bit ones.
-using IncSortConfig = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>,
-                                        rocprim::kernel_config<1024, 16>, 11,
-                                        rocprim::block_radix_rank_algorithm::match>>;
 
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
@@ -244,11 +233,9 @@ __global__ __launch_bounds__(256) void k_inc_sort(IncArgs a, int nsort)
 
 // Incidence lists from the neighbour-list slots (once per list). Slot (ii, jj) passes the
 // list's static filters of PackNeighborFunctor (cpp:84-94: rows past max_atoms, jj >= numneigh,
-// j >= max_atoms, the half filter j < i); its distance filter is applied each step from the
-// pack's validity bits. Atom a's list is its out-entries (the kept slots of its own row, in slot
-// order: other = j) followed by its in-entries (slots of other rows naming a: other = i, side
-// bit set) in ascending flat slot f = jj * rows + ii (the reference packer's flat order,
-// cpp:77-83). Only the in-entries need atomics and a sort; each row places its own out-entries.
+// j >= max_atoms, the half filter j < i); its distance filter is applied each step. Atom a's
+// list is its out-entries (the kept slots of its own row, in slot order: other = j) followed by
+// its in-entries (slots of other rows naming a: other = i, side bit set) in ascending i.
 struct ListArgs {
   const int *ilist;
   const int *numneigh;
@@ -258,15 +245,13 @@ struct ListArgs {
   int maxneighs;
   int max_atoms;
   int half_filter;
-  int pitch;  // row pitch of the validity bits
-  int *deg;
-  int *loc;
-  int *part;
-  uint32_t *tmp;
+  int *out_n;   // list slots of each atom's row (0: the atom is no row)
+  int *row_of;  // list row of each atom (-1: none)
+  int *loc;     // first entry of each atom
+  int *part;    // zero (loc holds whole offsets)
+  int *len;     // entries of each atom
   int *inc;
-  uint32_t *inc_bit;
-  int *len;
-  int fold;  // plain scheme: fold in-entries into the reverse out-entry (below)
+  int bin_log;  // atoms per bin: 1 << bin_log
 };
 
 // The row atom of list row ii and its slot count, or -1 when the row packs nothing.
@@ -286,15 +271,6 @@ __device__ __forceinline__ bool list_neighbor(const ListArgs &L, int i, int jj, 
   return !(L.half_filter && j < i);
 }
 
-// Validity-bit address of slot (ii, jj): word (jj >> 5) * pitch + ii, bit jj & 31.
-__device__ __forceinline__ uint32_t slot_bit(const ListArgs &L, int ii, int jj)
-{
-  return ((static_cast<uint32_t>(jj >> 5) * static_cast<uint32_t>(L.pitch) +
-           static_cast<uint32_t>(ii))
-          << 5) |
-         static_cast<uint32_t>(jj & 31);
-}
-
 // An in-entry (row i names atom a) whose reverse slot is one of a's out-entries (a's row names
 // i) gives a the same pair force in the plain scheme: the two slots pass the pack's distance
 // filter together (r^2 is the same sum of the negated differences), and a's plain-scheme share of
@@ -303,374 +279,466 @@ __device__ __forceinline__ uint32_t slot_bit(const ListArgs &L, int ii, int jj)
 // by the ends whose rows count. Each owned pair is then evaluated once per end instead of twice.
 constexpr uint32_t kIncPaired = 1u << 30;
 constexpr uint32_t kIncAtom = 0x3FFFFFFFu;
+constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 
 // ---------------------------------------------------------------------------------------------
-// The list-built incidence lists by one stable radix sort (once per list)
+// The list-built incidence lists through bins of atoms (once per list)
 // ---------------------------------------------------------------------------------------------
-// An atom's list is its out-entries (its own row's kept slots, in slot order) followed by its
-// in-entries (the kept slots of other rows that name it). The out-entries need no sorting: the
-// row's thread writes them. The in-entries are the kept slots keyed by the atom they name,
-// compacted row by row (row ii's slots in slot order, rows in list order) and radix-sorted by
-// that key; the sort is stable, so each atom's in-entries keep that row-major order: a
-// deterministic list without an atomic. With out[a] the out-entries of atom a and pre[a] their
-// prefix over the atoms below a, atom a's list starts at pre[a] + (in-entries of the atoms below
-// a: the sorted keys' lower bound of a), and the in-entry at sorted position p lands at
-// p + pre[a + 1].
+// The kept slots keyed by the atom they name are brought together in bins of 64 atoms (fewer for
+// rows too long for LDS): a count per bin, an exclusive scan, a scatter into the bins' ranges,
+// then one block per bin puts its atoms' lists together in LDS. The scatter's order inside a bin
+// follows atomic claims; the last pass orders each atom's in-entries by row atom, so the lists are
+// the same from run to run. The list is read four times, the entries written twice and read twice;
+// a radix sort of (atom, slot) pairs, the placing of out- and in-entries and the fold went over
+// the entries nine times: build of 256,000 atoms' half list (12.6 M entries) 566 -> 261 us,
+// of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
+constexpr int kBinLog = 6;
+constexpr int kBinAtoms = 1 << kBinLog;  // at most
+constexpr int kBinTiles = 8, kBinW = 2;  // a block's 64-row tiles and the waves of each
+constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
+constexpr int kBinProbes = 8;
 
-// One wave per 64-row tile (four per block): each lane counts its row's kept slots (the row
-// atom's out-entries); tilecnt[tile] = the tile's total, tilecnt[ntiles] = 0 so the scan's total
-// lands in the last offset.
-__global__ __launch_bounds__(256) void k_inc_tiles_count(ListArgs L, int ntiles,
-                                                         int *__restrict__ tilecnt)
+// An entry on its way: the atom's place in its bin above the row atom. 32 bits hold atoms below
+// 2^26 - 1.
+template <typename E>
+constexpr int kBinShift = sizeof(E) == 4 ? 26 : 32;
+constexpr long kBinAtoms32 = (1L << 26) - 1;
+
+// The bins' counters and offsets, [bins] each (offsets [bins + 1]).
+struct Bins {
+  int n;
+  int *next;  // in-entries, then the scatter's next free place
+  int *out;   // out-entries (list slots)
+  int *off;   // first in-entry in the scatter's output
+  int *loff;  // first entry in the lists
+};
+
+__global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
 {
-  const int tile = blockIdx.x * 4 + threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  if (tile > ntiles) return;  // whole wave
-  const int ii = tile * kWave + lane;
-  int c = 0;
-  if (tile < ntiles && ii < L.rows) {
-    int nn;
-    const int i = list_row(L, ii, nn);
-    if (i >= 0) {
-#pragma unroll 4
-      for (int jj = 0; jj < nn; ++jj) {
-        int j;
-        c += list_neighbor(L, i, jj, j) ? 1 : 0;
-      }
-      L.deg[i] = c;
-    }
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < L.max_atoms) {
+    L.out_n[i] = 0;
+    L.row_of[i] = -1;
   }
-  const int tot = wave_sum(c);
-  if (lane == 0) tilecnt[tile] = tot;
+  if (i < B.n) {
+    B.next[i] = 0;
+    B.out[i] = 0;
+  }
+  if (i < (L.max_atoms + kScanChunk) / kScanChunk) L.part[i] = 0;
 }
 
-// The in-entry keys (the atom a kept slot names) and values (the slot id f = jj * rows + ii),
-// tile by tile from the tile's offset, slot-major inside the tile: at each slot the wave's kept
-// entries are one contiguous run (ballot + rank), so the stores coalesce.
-__global__ __launch_bounds__(256) void k_inc_tiles_emit(ListArgs L, int ntiles,
-                                                        const int *__restrict__ tileoff,
-                                                        uint32_t *__restrict__ keys,
-                                                        uint32_t *__restrict__ vals)
+// Count (SCATTER false: the in- and out-entries of each bin; also out_n and row_of) and scatter.
+// One lane per row, the waves of a tile sharing its slots; entries of adjacent lanes in the same
+// bin (adjacent rows' k-th neighbours mostly are) count as one run, so a wave does one LDS update
+// per run.
+template <bool SCATTER, typename E>
+__global__ __launch_bounds__(kBinTiles *kBinW *kWave) LK_EIGHT_WAVES
+void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
 {
-  const int tile = blockIdx.x * 4 + threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  if (tile >= ntiles) return;  // whole wave
-  const int ii = tile * kWave + lane;
+  __shared__ int tag[kBinTable], cnt[kBinTable];
+  __shared__ int aux[kBinTable];  // count: out-entries; scatter: the block's first place
+  constexpr int kThreads = kBinTiles * kBinW * kWave;
+  const int wave = wave_in_block(), lane = threadIdx.x & (kWave - 1);
+  const int wq = wave % kBinW;
+  const int ii = (blockIdx.x * kBinTiles + wave / kBinW) * kWave + lane;
+  for (int k = threadIdx.x; k < kBinTable; k += kThreads) {
+    tag[k] = -1;
+    cnt[k] = 0;
+    aux[k] = 0;
+  }
   int nn = 0, i = -1;
   if (ii < L.rows) i = list_row(L, ii, nn);
   const int nmax = wave_max_int(nn);
-  int cursor = tileoff[tile];
-  for (int jj = 0; jj < nmax; ++jj) {
-    int j = 0;
-    const bool kept = jj < nn && list_neighbor(L, i, jj, j);
-    const uint64_t M = wave_ballot(kept);
-    if (kept) {
-      const int q = cursor + lanes_below(M);
-      keys[q] = static_cast<uint32_t>(j);
-      vals[q] = static_cast<uint32_t>(jj) * static_cast<uint32_t>(L.rows) +
-                static_cast<uint32_t>(ii);
+  __syncthreads();
+  // the LDS slot of bin b, or -1 when the probed slots hold other bins (they keep them: the same
+  // answer in both walks of the scatter)
+  auto slot_of = [&](int b) -> int {
+    uint32_t h = (static_cast<uint32_t>(b) * 2654435761u) >> 21;  // kBinTable = 2^11
+    for (int probe = 0; probe < kBinProbes; ++probe) {
+      int old = __hip_atomic_load(&tag[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (old == -1) old = atomicCAS(&tag[h], -1, b);
+      if (old == -1 || old == b) return static_cast<int>(h);
+      h = (h + 1) & (kBinTable - 1);
     }
-    cursor += __popcll(M);
+    return -1;
+  };
+  if (!SCATTER && wq == 0 && i >= 0) {
+    L.out_n[i] = nn;
+    L.row_of[i] = ii;
+    const int q = slot_of(i >> L.bin_log);
+    atomicAdd(q >= 0 ? &aux[q] : &B.out[i >> L.bin_log], nn);
   }
-}
-
-// first sorted position of key `k` (keys ascending, n entries)
-__device__ __forceinline__ int lower_bound_key(const uint32_t *keys, int n, uint32_t k)
-{
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = lo + ((hi - lo) >> 1);
-    if (keys[mid] < k) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// list offsets of atoms 0 .. atoms (inclusive); part[] stays zero (absolute offsets)
-__global__ __launch_bounds__(256) void k_inc_atoms_loc(const uint32_t *__restrict__ keys, int n,
-                                                       const int *__restrict__ pre, int atoms,
-                                                       int *__restrict__ loc)
-{
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a > atoms) return;
-  loc[a] = pre[a] + lower_bound_key(keys, n, static_cast<uint32_t>(a));
-}
-
-// out-entries, one thread per row: the neighbour and the slot's validity-bit address
-__global__ __launch_bounds__(256) void k_inc_rows_place(ListArgs L)
-{
-  const int ii = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ii >= L.rows) return;
-  int nn;
-  const int i = list_row(L, ii, nn);
-  if (i < 0) return;
-  int q = L.loc[i];
-  for (int jj = 0; jj < nn; ++jj) {
-    int j;
-    if (!list_neighbor(L, i, jj, j)) continue;
-    L.inc[q] = j;
-    L.inc_bit[q] = slot_bit(L, ii, jj);
-    ++q;
-  }
-}
-
-// Out-entries through LDS, one wave (block) per 64-row tile: each lane stages its row's kept
-// neighbours (and their slot numbers) in LDS, a row to `pitch` entries (odd: no bank conflicts),
-// then the wave writes the rows one after another, 64 consecutive entries per store. The list is
-// read slot-major and the lists written atom-major, both coalesced. Eight list slots per lane are
-// loaded before any is used, so eight loads of each wave are in flight.
-__global__ __launch_bounds__(kWave) void k_inc_tiles_place(ListArgs L, int ntiles, int pitch)
-{
-  extern __shared__ int stage[];  // [64][pitch] neighbours, then [64][pitch] slot numbers (u8)
-  const int tile = blockIdx.x;
-  const int lane = threadIdx.x;
-  if (tile >= ntiles) return;
-  const int ii = tile * kWave + lane;
-  int nn = 0, i = -1;
-  if (ii < L.rows) i = list_row(L, ii, nn);
-  int *sj = stage + lane * pitch;
-  unsigned char *sq = reinterpret_cast<unsigned char *>(stage + kWave * pitch) + lane * pitch;
-  const int base_own = i >= 0 ? L.loc[i] : 0;  // loaded with the list, not inside the row loop
-  int c = 0;
-  constexpr int kBatch = 8;
-  for (int j0 = 0; j0 < nn; j0 += kBatch) {
-    int raw[kBatch];
+  auto walk = [&](auto &&use) {
+    constexpr int kBatch = 8;
+    for (int j0 = wq; j0 < nmax; j0 += kBinW * kBatch) {
+      int raw[kBatch];
 #pragma unroll
-    for (int q = 0; q < kBatch; ++q)
-      raw[q] = j0 + q < nn ? L.neighbors[static_cast<long>(j0 + q) * L.stride + i] : 0;
+      for (int u = 0; u < kBatch; ++u) {
+        const int jj = j0 + kBinW * u;
+        raw[u] = jj < nn ? L.neighbors[static_cast<long>(jj) * L.stride + i] : 0;
+      }
 #pragma unroll
-    for (int q = 0; q < kBatch; ++q) {
-      const int j = raw[q] & kNeighMask;
-      // list_neighbor's filter on the loaded entry
-      if (j0 + q < nn && j < L.max_atoms && !(L.half_filter && j < i)) {
-        sj[c] = j;
-        sq[c] = static_cast<unsigned char>(j0 + q);
-        ++c;
+      for (int u = 0; u < kBatch; ++u) {
+        if (j0 + kBinW * u >= nmax) break;  // wave-uniform
+        const int j = raw[u] & kNeighMask;
+        // list_neighbor's filter on the loaded entry
+        const bool ok = j0 + kBinW * u < nn && j < L.max_atoms && !(L.half_filter && j < i);
+        const int b = ok ? j >> L.bin_log : -1;
+        const int before = __shfl_up(b, 1, kWave);
+        const bool head = lane == 0 || before != b;
+        const uint64_t heads = wave_ballot(head);
+        const uint64_t upto = (2ull << lane) - 1ull;  // lanes up to this one
+        const uint64_t next = heads & ~upto;
+        const int n = (next ? __builtin_ctzll(next) : kWave) - lane;  // a head's run
+        use(j, b, head, n, 63 - __builtin_clzll(heads & upto));
       }
     }
+  };
+  walk([&](int, int b, bool head, int n, int) {
+    if (!head || b < 0) return;
+    const int q = slot_of(b);
+    if (q >= 0)
+      atomicAdd(&cnt[q], n);
+    else if (!SCATTER)
+      atomicAdd(&B.next[b], n);
+  });
+  __syncthreads();
+  for (int k = threadIdx.x; k < kBinTable; k += kThreads) {
+    if (tag[k] < 0) continue;
+    if constexpr (SCATTER) {
+      if (cnt[k] == 0) continue;
+      aux[k] = atomicAdd(&B.next[tag[k]], cnt[k]);
+      cnt[k] = 0;
+    } else {
+      if (cnt[k]) atomicAdd(&B.next[tag[k]], cnt[k]);
+      if (aux[k]) atomicAdd(&B.out[tag[k]], aux[k]);
+    }
+  }
+  if constexpr (SCATTER) {
+    __syncthreads();
+    walk([&](int j, int b, bool head, int n, int first) {
+      int at = 0;
+      if (head && b >= 0) {
+        const int q = slot_of(b);
+        at = q >= 0 ? aux[q] + atomicAdd(&cnt[q], n) : atomicAdd(&B.next[b], n);
+      }
+      at = __shfl(at, first, kWave) + lane - first;
+      if (b >= 0)
+        tmp[at] = (static_cast<E>(j & ((1 << L.bin_log) - 1)) << kBinShift<E>) | static_cast<E>(i);
+    });
+  }
+}
+
+// Exclusive scans of the bins' in-entries (off, and next in place) and of all their entries (loff),
+// one block.
+__global__ __launch_bounds__(kScanThreads) void k_inc_bin_scan(Bins B)
+{
+  __shared__ int wsum[2][kScanThreads / kWave];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  int carry = 0, carry_l = 0;
+  for (int b0 = 0; b0 < B.n; b0 += kScanChunk) {
+    int v[kScanItems], w[kScanItems], s = 0, sl = 0;
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+      const int k = b0 + t * kScanItems + q;
+      v[q] = k < B.n ? B.next[k] : 0;
+      w[q] = k < B.n ? v[q] + B.out[k] : 0;
+      s += v[q];
+      sl += w[q];
+    }
+    int incl = s, incl_l = sl;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int y = __shfl_up(incl, o, kWave), yl = __shfl_up(incl_l, o, kWave);
+      if (lane >= o) {
+        incl += y;
+        incl_l += yl;
+      }
+    }
+    if (lane == kWave - 1) {
+      wsum[0][wave] = incl;
+      wsum[1][wave] = incl_l;
+    }
+    __syncthreads();
+    int run = carry + incl - s, run_l = carry_l + incl_l - sl;
+    for (int q = 0; q < kScanThreads / kWave; ++q) {
+      run += q < wave ? wsum[0][q] : 0;
+      run_l += q < wave ? wsum[1][q] : 0;
+      carry += wsum[0][q];
+      carry_l += wsum[1][q];
+    }
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+      const int k = b0 + t * kScanItems + q;
+      if (k < B.n) {
+        B.next[k] = run;
+        B.off[k] = run;
+        B.loff[k] = run_l;
+      }
+      run += v[q];
+      run_l += w[q];
+    }
+    __syncthreads();
+  }
+  if (t == 0) B.off[B.n] = carry;
+}
+
+__device__ __forceinline__ uint32_t bin_hash(uint32_t atom, uint32_t slots)
+{
+  return static_cast<uint32_t>((static_cast<uint64_t>(atom * 2654435761u) * slots) >> 32);
+}
+
+// Values below v among the `n4` groups of four at `v4`. TIES: values equal to v before index `at`
+// count too, so that equal values (a list that names an atom twice) take places of their own.
+template <bool TIES>
+__device__ __forceinline__ int rank_of(const uint4 *v4, int n4, uint32_t v, int at)
+{
+  int rank = 0;
+  for (int m = 0; m < n4; ++m) {
+    const uint4 q = v4[m];
+    rank += (q.x < v ? 1 : 0) + (q.y < v ? 1 : 0) + (q.z < v ? 1 : 0) + (q.w < v ? 1 : 0);
+    if (TIES)
+      rank += (q.x == v && 4 * m + 0 < at ? 1 : 0) + (q.y == v && 4 * m + 1 < at ? 1 : 0) +
+              (q.z == v && 4 * m + 2 < at ? 1 : 0) + (q.w == v && 4 * m + 3 < at ? 1 : 0);
+  }
+  return rank;
+}
+
+// One wave stores the `c` values of slots[0, n) below 2^31 (`n` a multiple of four) in ascending
+// order, the side bit set. Distinct values have the ranks 0 .. c - 1, which sum to c (c - 1) / 2;
+// any other sum means equal ones, and the ranks are taken again with ties broken.
+__device__ __forceinline__ void store_ranked(const uint32_t *slots, int n, int c, int *out)
+{
+  const uint4 *v4 = reinterpret_cast<const uint4 *>(slots);
+  const int lane = threadIdx.x & (kWave - 1);
+  int sum = 0;
+  for (int q = lane; q < n; q += kWave) {
+    const uint32_t v = slots[q];
+    if (v >> 31) continue;
+    const int r = rank_of<false>(v4, n / 4, v, q);
+    out[r] = static_cast<int>(v | (1u << 31));
+    sum += r;
+  }
+  if (wave_sum(sum) == c * (c - 1) / 2) return;
+  for (int q = lane; q < n; q += kWave) {
+    const uint32_t v = slots[q];
+    if (v >> 31) continue;
+    out[rank_of<true>(v4, n / 4, v, q)] = static_cast<int>(v | (1u << 31));
+  }
+}
+
+// One block per bin: the lists of its atoms. Their out-entries are staged in LDS, `pitch` slots per
+// atom (odd: no bank conflicts), and their in-entries meet in `per_atom` slots per atom: for
+// the half scheme as segments, for the plain one as hash tables of row atoms, in which the
+// out-entries look up their reverse (one that finds it is marked, and the in-entry leaves). The
+// out-entries are written without their gaps, what is left of the in-entries ranked by row atom.
+// A bin whose in-entries do not fit (and every bin when per_atom is 0) searches its rows and
+// entries in memory instead.
+constexpr int kListThreads = 1024;
+
+template <typename E, bool FOLD>
+__global__ __launch_bounds__(kListThreads) LK_EIGHT_WAVES
+void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int per_atom, int pitch)
+{
+  extern __shared__ __align__(16) uint32_t pool[];  // [atoms][per_atom], then [atoms][pitch]
+  __shared__ int nin[kBinAtoms], nout[kBinAtoms], rown[kBinAtoms];
+  __shared__ int start[kBinAtoms], seg[kBinAtoms], next[kBinAtoms];
+  __shared__ int spill;
+  constexpr int kWaves = kListThreads / kWave;
+  const int tid = threadIdx.x, wave = wave_in_block(), lane = tid & (kWave - 1);
+  const int na = 1 << L.bin_log, a0 = blockIdx.x << L.bin_log;
+  const int e0 = B.off[blockIdx.x], n = B.off[blockIdx.x + 1] - e0;
+  const int slots = na * per_atom;
+  uint32_t *outs = pool + slots;
+  auto atom_of = [](E v) { return static_cast<int>(v >> kBinShift<E>); };
+  auto row_atom = [](E v) {
+    return static_cast<uint32_t>(v & ((static_cast<E>(1) << kBinShift<E>) - 1));
+  };
+  if (tid < kBinAtoms) {
+    nin[tid] = 0;
+    nout[tid] = 0;
+    next[tid] = 0;
+    rown[tid] = tid < na && a0 + tid < L.max_atoms ? L.out_n[a0 + tid] : 0;
+  }
+  if (tid == 0) spill = per_atom == 0;
+  for (int k = tid; k < slots; k += kListThreads) pool[k] = kIncNone;
+  __syncthreads();
+  // the places of the atoms' lists from their counts, by the first wave
+  auto place = [&]() {
+    if (wave == 0) {
+      const int c4 = (nin[lane] + 3) & ~3, c = nin[lane] + nout[lane];
+      int incl = c, incl4 = c4;
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int y = __shfl_up(incl, o, kWave), y4 = __shfl_up(incl4, o, kWave);
+        if (lane >= o) {
+          incl += y;
+          incl4 += y4;
+        }
+      }
+      start[lane] = B.loff[blockIdx.x] + incl - c;
+      seg[lane] = incl4 - c4;
+      if (!FOLD && incl4 > slots) spill = 1;  // the half scheme's segments
+      if (lane < na && a0 + lane < L.max_atoms) {
+        L.loc[a0 + lane] = start[lane];
+        L.len[a0 + lane] = c;
+      }
+    }
+    __syncthreads();
+  };
+  // thread t stages the slots t / na, + threads / na, ... of atom t % na
+  const int d_own = tid & (na - 1), q0 = tid >> L.bin_log, qstep = kListThreads >> L.bin_log;
+  if (per_atom > 0) {
+    if constexpr (FOLD) {
+      for (int e = tid; e < n; e += kListThreads) {
+        const E v = tmp[e0 + e];
+        uint32_t *keys = pool + atom_of(v) * per_atom;
+        uint32_t h = bin_hash(row_atom(v), per_atom);
+        bool in = false;
+        for (int probe = 0; probe < per_atom && !in; ++probe) {
+          in = atomicCAS(&keys[h], kIncNone, row_atom(v)) == kIncNone;
+          if (++h == static_cast<uint32_t>(per_atom)) h = 0;
+        }
+        if (!in) spill = 1;
+      }
+      __syncthreads();
+    } else {
+      for (int e = tid; e < n; e += kListThreads) atomicAdd(&nin[atom_of(tmp[e0 + e])], 1);
+    }
+    uint32_t *keys = pool + d_own * per_atom;
+    for (int b0 = q0; b0 < rown[d_own]; b0 += 4 * qstep) {
+      int raw[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int jj = b0 + u * qstep;
+        raw[u] = jj < rown[d_own]
+                     ? L.neighbors[static_cast<long>(jj) * L.stride + a0 + d_own] & kNeighMask
+                     : INT_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int jj = b0 + u * qstep, j = raw[u];
+        if (jj >= rown[d_own]) break;
+        uint32_t v = static_cast<uint32_t>(j);
+        if (j >= L.max_atoms || (L.half_filter && j < a0 + d_own)) {
+          v = kIncNone;  // list_neighbor's filter
+        } else if constexpr (FOLD) {
+          uint32_t h = bin_hash(v, per_atom);
+          for (int probe = 0; probe < per_atom; ++probe) {
+            const uint32_t k = keys[h];
+            if (k == kIncNone) break;
+            if (k == static_cast<uint32_t>(j) && !(atomicOr(&keys[h], 1u << 31) >> 31)) {
+              v |= kIncPaired;
+              break;
+            }
+            if (++h == static_cast<uint32_t>(per_atom)) h = 0;
+          }
+        }
+        outs[d_own * pitch + jj] = v;
+      }
+    }
+    __syncthreads();
+    for (int d = wave; d < na; d += kWaves) {
+      int c = 0, ci = 0;
+      for (int k = 0; k < rown[d]; k += kWave)
+        c += __popcll(wave_ballot(k + lane < rown[d] && outs[d * pitch + k + lane] != kIncNone));
+      if (FOLD)
+        for (int k = 0; k < per_atom; k += kWave)
+          ci += __popcll(wave_ballot(k + lane < per_atom && !(pool[d * per_atom + k + lane] >> 31)));
+      if (lane == 0) {
+        nout[d] = c;
+        if (FOLD) nin[d] = ci;
+      }
+    }
+    __syncthreads();
+    const bool fits = !FOLD || !spill;
+    if (fits) place();
+    if (fits && !spill) {
+      if constexpr (!FOLD) {
+        for (int e = tid; e < n; e += kListThreads) {
+          const E v = tmp[e0 + e];
+          const int d = atom_of(v);
+          pool[seg[d] + atomicAdd(&next[d], 1)] = row_atom(v);
+        }
+        __syncthreads();
+      }
+      for (int d = wave; d < na; d += kWaves) {
+        int *to = L.inc + start[d];
+        for (int k = 0; k < rown[d]; k += kWave) {
+          const uint32_t v = k + lane < rown[d] ? outs[d * pitch + k + lane] : kIncNone;
+          const uint64_t M = wave_ballot(v != kIncNone);
+          if (v != kIncNone) to[lanes_below(M)] = static_cast<int>(v);
+          to += __popcll(M);
+        }
+        if (nin[d] > 0)
+          store_ranked(FOLD ? pool + d * per_atom : pool + seg[d],
+                       FOLD ? per_atom : (nin[d] + 3) & ~3, nin[d], to);
+      }
+      return;
+    }
+    if (tid < kBinAtoms) {
+      nin[tid] = 0;
+      nout[tid] = 0;
+    }
+    __syncthreads();
+  }
+  // In memory. An in-entry is folded when its row atom is one of the atom's out-entries; the first
+  // such out-entry is marked.
+  auto folded = [&](E v) -> bool {
+    if (!FOLD) return false;
+    const int d = atom_of(v);
+    for (int jj = 0; jj < rown[d]; ++jj) {
+      int j;
+      if (list_neighbor(L, a0 + d, jj, j) && static_cast<uint32_t>(j) == row_atom(v)) return true;
+    }
+    return false;
+  };
+  for (int jj = q0; jj < rown[d_own]; jj += qstep) {
+    int j;
+    if (list_neighbor(L, a0 + d_own, jj, j)) atomicAdd(&nout[d_own], 1);
+  }
+  for (int e = tid; e < n; e += kListThreads)
+    if (!folded(tmp[e0 + e])) atomicAdd(&nin[atom_of(tmp[e0 + e])], 1);
+  __syncthreads();
+  place();
+  for (int jj = q0; jj < rown[d_own]; jj += qstep) {
+    int j, before = 0;
+    if (!list_neighbor(L, a0 + d_own, jj, j)) continue;
+    bool paired = FOLD;
+    for (int k = 0; k < jj; ++k) {
+      int jk;
+      if (!list_neighbor(L, a0 + d_own, k, jk)) continue;
+      ++before;
+      if (jk == j) paired = false;
+    }
+    if (paired) {
+      paired = false;
+      for (int e = 0; e < n && !paired; ++e)
+        paired = atom_of(tmp[e0 + e]) == d_own && row_atom(tmp[e0 + e]) == static_cast<uint32_t>(j);
+    }
+    L.inc[start[d_own] + before] = static_cast<int>(static_cast<uint32_t>(j) |
+                                                    (paired ? kIncPaired : 0u));
   }
   __syncthreads();
-  for (int r = 0; r < kWave; ++r) {
-    const int cr = __shfl(c, r, kWave);
-    if (cr == 0) continue;  // wave-uniform
-    const int base = __shfl(base_own, r, kWave);
-    const int *rj = stage + r * pitch;
-    const unsigned char *rq = reinterpret_cast<const unsigned char *>(stage + kWave * pitch) + r * pitch;
-    for (int k = lane; k < cr; k += kWave) {
-      L.inc[base + k] = rj[k];
-      L.inc_bit[base + k] = slot_bit(L, tile * kWave + r, rq[k]);
-    }
-  }
-}
-
-// Out-entries through LDS, one wave (block) per 64-row tile, staged compactly: the tile's kept
-// entries in row order, each row's run at the prefix of the rows' out-entry counts, with the row
-// of each entry beside it; then 64 staged entries per store, each to its row's list at its place
-// in the run. A round stages the rows whose runs fit `cap` entries together (one row always
-// fits: cap >= maxneighs); rows past that wait for the next round. The list is read slot-major
-// (eight slots per lane in flight) and the lists written atom-major, both coalesced; sized to
-// the mean run rather than the longest row, the staging leaves more waves per CU when the rows
-// are ragged, and each store writes 64 entries however the rows end.
-__global__ __launch_bounds__(kWave) void k_inc_tiles_place_runs(ListArgs L, int ntiles, int cap)
-{
-  extern __shared__ int stage[];  // [cap] neighbours, [64] run starts, [64] list bases, then
-                                  // [cap] slot numbers (u8), [cap] rows (u8)
-  const int tile = blockIdx.x;
-  const int lane = threadIdx.x;
-  if (tile >= ntiles) return;
-  int *sj = stage;
-  int *rstart = stage + cap;
-  int *rbase = rstart + kWave;
-  unsigned char *sq = reinterpret_cast<unsigned char *>(rbase + kWave);
-  unsigned char *sr = sq + cap;
-  const int ii = tile * kWave + lane;
-  int nn = 0, i = -1;
-  if (ii < L.rows) i = list_row(L, ii, nn);
-  const int c = i >= 0 ? L.deg[i] : 0;  // kept out-entries (k_inc_tiles_count)
-  const int base_own = i >= 0 ? L.loc[i] : 0;
-  int incl = c;  // inclusive prefix of the counts over the tile's rows
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const int v = __shfl_up(incl, off, kWave);
-    if (lane >= off) incl += v;
-  }
-  int r0 = 0, staged_before = 0;  // wave-uniform
-  while (r0 < kWave) {
-    const int start = incl - c - staged_before;  // this row's run in this round
-    const uint64_t F = wave_ballot(lane >= r0 && start + c <= cap);
-    const int r1 = 64 - __clzll(F);  // rows r0 .. r1 - 1 (the prefix is nondecreasing)
-    const bool mine = lane >= r0 && lane < r1;
-    if (mine) {
-      rstart[lane] = start;
-      rbase[lane] = base_own;
-      int k = start;
-      constexpr int kBatch = 8;
-      for (int j0 = 0; j0 < nn; j0 += kBatch) {
-        int raw[kBatch];
-#pragma unroll
-        for (int q = 0; q < kBatch; ++q)
-          raw[q] = j0 + q < nn ? L.neighbors[static_cast<long>(j0 + q) * L.stride + i] : 0;
-#pragma unroll
-        for (int q = 0; q < kBatch; ++q) {
-          const int j = raw[q] & kNeighMask;
-          // list_neighbor's filter on the loaded entry
-          if (j0 + q < nn && j < L.max_atoms && !(L.half_filter && j < i)) {
-            sj[k] = j;
-            sq[k] = static_cast<unsigned char>(j0 + q);
-            sr[k] = static_cast<unsigned char>(lane);
-            ++k;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    const int total = __shfl(incl, r1 - 1, kWave) - staged_before;
-    for (int e = lane; e < total; e += kWave) {
-      const int r = sr[e];
-      const int q = rbase[r] + (e - rstart[r]);
-      L.inc[q] = sj[e];
-      L.inc_bit[q] = slot_bit(L, tile * kWave + r, sq[e]);
-    }
-    __syncthreads();
-    staged_before += total;
-    r0 = r1;
-  }
-}
-
-// keys of the sort's unused tail [kept, n) (kept read on the device): the pad key, above every atom
-__global__ __launch_bounds__(256) void k_inc_pad_keys(uint32_t *__restrict__ keys,
-                                                      const int *__restrict__ kept, int n,
-                                                      uint32_t pad)
-{
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n && p >= *kept) keys[p] = pad;
-}
-
-// in-entries, one thread per sorted position: the row atom with the side bit, and the slot's
-// validity-bit address
-__global__ __launch_bounds__(256) void k_inc_sorted_place(ListArgs L,
-                                                          const uint32_t *__restrict__ keys,
-                                                          const uint32_t *__restrict__ vals, int n,
-                                                          const int *__restrict__ pre)
-{
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const uint32_t key = keys[p];
-  if (key >= static_cast<uint32_t>(L.max_atoms)) return;  // the pad of an unused tail
-  const int a = static_cast<int>(key);
-  const uint32_t f = vals[p];
-  const int ii = static_cast<int>(f % static_cast<uint32_t>(L.rows));
-  const int jj = static_cast<int>(f / static_cast<uint32_t>(L.rows));
-  const int q = p + pre[a + 1];
-  L.inc[q] = static_cast<int>(static_cast<uint32_t>(L.ilist[ii]) | (1u << 31));
-  L.inc_bit[q] = slot_bit(L, ii, jj);
-}
-
-constexpr int kFoldLanes = 16;    // lanes per atom in the fold
-constexpr int kFoldSlots = 256;   // LDS hash slots per atom: up to kFoldSlots / 2 out-entries
-
-__device__ __forceinline__ int fold_slot(int atom)
-{
-  return static_cast<int>((static_cast<uint32_t>(atom) * 0x9E3779B1u) >> 24);
-}
-
-// Plain scheme only, after the lists are placed: the fold above (an in-entry whose row atom is
-// also one of the atom's out-entries is dropped and the first such out-entry marked), then the
-// kept in-entries close up in order; len[a] = the list's length. Sixteen lanes per atom, sixteen
-// atoms per block. When every atom of the block has at most kFoldSlots / 2 out-entries, each atom's
-// out-entries go into an open-addressing table in LDS (partner atom -> lowest out index) and each
-// in-entry probes it; otherwise the in-entries are compared against every out-entry by shuffles,
-// with the loops run to the wave's longest list so every shuffle reads an active lane.
-__global__ __launch_bounds__(256) void k_inc_list_fold_sorted(ListArgs L, int natoms)
-{
-  constexpr int G = kFoldLanes;
-  __shared__ int keys[256 / G][kFoldSlots];
-  __shared__ int first[256 / G][kFoldSlots];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int g = lane / G, gl = lane % G, grp = threadIdx.x / G;
-  const int atom = blockIdx.x * (256 / G) + grp;
-  const bool have = atom < natoms;
-  int b0 = 0, out = 0, len = 0;
-  if (have) {
-    b0 = inc_off(L.loc, L.part, atom);
-    out = L.deg[atom];
-    len = inc_off(L.loc, L.part, atom + 1) - b0 - out;
-  }
-  const int b = b0 + out;
-  const bool hashed = !__syncthreads_or(out > kFoldSlots / 2);  // block-uniform
-  if (hashed) {
-    for (int i = gl; i < kFoldSlots; i += G) {
-      keys[grp][i] = -1;
-      first[grp][i] = INT_MAX;
-    }
-    __syncthreads();
-    for (int c = gl; c < out; c += G) {
-      const int w = static_cast<int>(static_cast<uint32_t>(L.inc[b0 + c]) & kIncAtom);
-      int h = fold_slot(w);
-      // at most half the slots are taken, so an empty or matching slot is always reached
-      for (int t = 0; t < kFoldSlots; ++t) {
-        const int old = atomicCAS(&keys[grp][h], -1, w);
-        if (old == -1 || old == w) {
-          atomicMin(&first[grp][h], c);
-          break;
-        }
-        h = (h + 1) & (kFoldSlots - 1);
-      }
-    }
+  // the folded entries become all ones (no entry is: its row atom is below 2^26 - 1, or 2^30 in
+  // 64 bits), so that the ranks below see the others alone
+  constexpr E kGone = ~static_cast<E>(0);
+  if constexpr (FOLD) {
+    for (int e = tid; e < n; e += kListThreads)
+      if (folded(tmp[e0 + e])) tmp[e0 + e] = kGone;
+    __threadfence();
     __syncthreads();
   }
-  const int len_max = wave_max_int(len), out_max = wave_max_int(out);
-  if (len_max == 0) {  // whole wave
-    if (have && gl == 0) L.len[atom] = out;
-    return;
+  for (int e = tid; e < n; e += kListThreads) {
+    const E v = tmp[e0 + e];
+    if (v == kGone) continue;
+    int r = 0;
+    for (int m = 0; m < n; ++m) {
+      const E w = tmp[e0 + m];
+      r += atom_of(w) == atom_of(v) && w != kGone && (w < v || (w == v && m < e)) ? 1 : 0;
+    }
+    L.inc[start[atom_of(v)] + nout[atom_of(v)] + r] = static_cast<int>(row_atom(v) | (1u << 31));
   }
-  int kept = 0;
-  for (int c0 = 0; c0 < len_max; c0 += G) {
-    const bool mine = c0 + gl < len;
-    int row_atom = -1;
-    uint32_t bit = 0;
-    if (mine) {
-      row_atom = static_cast<int>(static_cast<uint32_t>(L.inc[b + c0 + gl]) & kIncAtom);
-      bit = L.inc_bit[b + c0 + gl];
-    }
-    int hit = -1;
-    if (hashed) {
-      if (mine) {
-        int h = fold_slot(row_atom);
-        for (int t = 0; t < kFoldSlots; ++t) {
-          const int k = keys[grp][h];
-          if (k == row_atom) {
-            hit = first[grp][h];
-            break;
-          }
-          if (k < 0) break;
-          h = (h + 1) & (kFoldSlots - 1);
-        }
-      }
-    } else {
-      for (int c1 = 0; c1 < out_max; c1 += G) {
-        const int w = c1 + gl < out ? static_cast<int>(L.inc[b0 + c1 + gl] & kIncAtom) : -2;
-#pragma unroll
-        for (int m = 0; m < G; ++m) {
-          const int wm = __shfl(w, g * G + m, kWave);
-          if (hit < 0 && wm == row_atom) hit = c1 + m;
-        }
-      }
-    }
-    // every lane has read the chunk (row_atom, bit) before any write below, and a kept entry
-    // moves to a position no later than its own, so the close-up is safe in place
-    if (mine && hit >= 0)
-      L.inc[b0 + hit] = static_cast<int>(static_cast<uint32_t>(row_atom) | kIncPaired);
-    const bool keep = mine && hit < 0;
-    const uint64_t M = (wave_ballot(keep) >> (g * G)) & 0xFFFFull;
-    if (keep) {
-      const int q = b + kept + __popcll(M & ((1ull << gl) - 1ull));
-      L.inc[q] = static_cast<int>(static_cast<uint32_t>(row_atom) | (1u << 31));
-      L.inc_bit[q] = bit;
-    }
-    kept += __popcll(M);
-  }
-  if (have && gl == 0) L.len[atom] = out + kept;
 }
 
 template <int G, typename T>
@@ -686,7 +754,7 @@ struct TwoSided {
   const int *loc;
   const int *part;
   const int *inc;
-  const int *len;  // entries of each atom's list when the build folded pairs, else null
+  const int *len;  // entries of each atom
   int nall;
   int nlocal;
   int nadd;             // rows that take the force add: nall with newton on, else nlocal
@@ -696,24 +764,16 @@ struct TwoSided {
   const int *ghost_off;
   const int *ghost_list;
   int nblk;             // 64-atom partial tiles over nall
-  const uint32_t *inc_bit;  // list-built entries: address of the slot's validity bit
-  const uint32_t *bits;     // the pack's validity bits of this step
+  const uint32_t *bits;     // kFromBits: the pack's validity bits by list row, and the list
+  const int *row_of, *out_n;  // each atom's list row and its slots
+  const int *neighbors;
+  long stride;
+  int max_atoms;
   double cutsq_pack;        // the pack's filter: rsq <= cutsq in float64 (cpp:91)
   float cutsq_lo, cutsq_hi; // cutsq_pack rounded down and up to float
   const int *ghost_flag;    // 1 when a packed edge starts on a ghost row (the pack's flag)
   FusedPack pack;           // a fused pack of this step: tail reset and counts (else unused)
 };
-
-// Entries of atom a's list starting at b: all of its range, less the in-entries a fold dropped.
-__device__ __forceinline__ int inc_len(const TwoSided &t, int a, int b)
-{
-  return t.len ? t.len[a] : inc_off(t.loc, t.part, a + 1) - b;
-}
-
-__device__ __forceinline__ bool word_has(uint32_t word, uint32_t ba)
-{
-  return ((word >> (ba & 31u)) & 1u) != 0;
-}
 
 // Whether the pack kept an entry's list slot this step, decided from the entry's own geometry
 // wherever that decides it, so the sweeps gather no validity word. The pack keeps rsq <= cutsq,
@@ -727,12 +787,13 @@ __device__ __forceinline__ bool word_has(uint32_t word, uint32_t ba)
 // |sum d^2 - sum D^2| <= sum b_c (2|d_c| + b_c) <= u s (2 l1 + u s) / (1 - u)^2, and r2 is within
 // 3u r2 / (1 - 3u) of sum d^2 (float64 rounding adds far less). band = 2u (s (2 l1 + u s) + 4 r2),
 // computed in float, exceeds twice that bound and at least 8u r2, which covers the rounding of
-// r2 +- band against cutsq rounded down (up) to float. Only an r2 inside the band loads the
-// bit address of entry q's slot and then its validity word; no other entry reads either. Per
-// row, BandRow bounds the band of every entry the model's cutoff lets through (l1 <= sqrt(3)
+// r2 +- band against cutsq rounded down (up) to float. Only an r2 inside the band looks further:
+// where the pack ran in this call it forms rsq from the engine's positions as the pack did (the
+// sign of the differences does not matter), else it finds the entry's slot in its sender's row and
+// reads that slot's validity bit. Per row, BandRow bounds the band of every entry the model's cutoff lets through (l1 <= sqrt(3)
 // rc_model, and the neighbour's 1-norm <= the row's + l1), so most entries are decided by one
-// comparison with a row threshold. Lists built from packed edges (no bit addresses) hold kept
-// slots only.
+// comparison with a row threshold. Lists built from packed edges hold kept slots only (no
+// filter).
 template <typename S>
 struct BandRow {
   S sa;       // the row atom's 1-norm
@@ -756,13 +817,42 @@ __device__ __forceinline__ BandRow<S> band_row(const TwoSided &t, const Atom4<S>
   return br;
 }
 
-template <typename S>
-__device__ __forceinline__ bool slot_kept(const TwoSided &t, int q, S r2, S dx, S dy, S dz,
-                                          const BandRow<S> &br, const Atom4<S> &xo)
+// How a sweep tells the kept entries, a template parameter of the sweeps: inside the band from
+// the positions of this call's pack, or from the validity bits of an earlier one. (Both in one
+// kernel held 94 SGPRs in the float32 density sweep: one block per CU, 59 -> 71 us at 256,000 atoms.)
+enum Filter { kAllKept = 0, kFromX = 1, kFromBits = 2 };
+
+// The decision inside the band: atom a's entry with atom o, on o's row when `in`.
+template <int FILTER>
+__device__ __forceinline__ bool kept_by_pack(const TwoSided &t, int a, int o, bool in)
 {
-  if (!t.inc_bit) return true;
+  if constexpr (FILTER == kFromX) {
+#pragma clang fp contract(off)
+    double rsq = 0.0;
+#pragma unroll 1  // rare: few registers before few instructions
+    for (int c = 0; c < 3; ++c) {
+      const double d = t.x[3L * a + c] - t.x[3L * o + c];
+      rsq = rsq + d * d;
+    }
+    return !(rsq > t.cutsq_pack);
+  } else {
+    const int snd = in ? o : a, rcv = in ? a : o;
+    const int ii = t.row_of[snd], nn = t.out_n[snd];
+    for (int jj = 0; jj < nn; ++jj)
+      if ((t.neighbors[static_cast<long>(jj) * t.stride + snd] & kNeighMask) == rcv)
+        return ((t.bits[static_cast<long>(jj >> 5) * t.max_atoms + ii] >> (jj & 31)) & 1u) != 0;
+    return false;
+  }
+}
+
+template <int FILTER, typename S>
+__device__ __forceinline__ bool slot_kept(const TwoSided &t, int a, uint32_t v, S r2, S dx, S dy,
+                                          S dz, const BandRow<S> &br, const Atom4<S> &xo)
+{
+  if constexpr (FILTER == kAllKept) return true;
   if constexpr (sizeof(S) == 8) {
-    (void)q;
+    (void)a;
+    (void)v;
     (void)dx;
     (void)dy;
     (void)dz;
@@ -778,8 +868,7 @@ __device__ __forceinline__ bool slot_kept(const TwoSided &t, int q, S r2, S dx, 
     const float band = 2.0f * u * (s * (2.0f * l1 + u * s) + 4.0f * r2);
     if (r2 + band <= t.cutsq_lo) return true;
     if (r2 - band > t.cutsq_hi) return false;
-    const uint32_t ba = t.inc_bit[q];
-    return word_has(t.bits[ba >> 5], ba);
+    return kept_by_pack<FILTER>(t, a, static_cast<int>(v & kIncAtom), (v >> 31) != 0);
   }
 }
 
@@ -793,7 +882,6 @@ __device__ __forceinline__ bool slot_kept(const TwoSided &t, int q, S r2, S dx, 
 template <int G>
 struct IncCursor {
   uint32_t v = 0;
-  int q = 0;  // the entry v was loaded from
   int b, last;
   __device__ __forceinline__ IncCursor(const TwoSided &t, int b_, int L, int gl) : b(b_), last(b_ + L - 1)
   {
@@ -802,7 +890,6 @@ struct IncCursor {
   __device__ __forceinline__ void load(const TwoSided &t, int q_)
   {
     v = static_cast<uint32_t>(t.inc[q_]);
-    q = q_;
   }
   __device__ __forceinline__ void advance(const TwoSided &t, int k)
   {
@@ -831,10 +918,9 @@ __device__ __forceinline__ S geometry(const Atom4<S> &xa, const Atom4<S> &xo, S 
 // Density per row (eam.py:298-314); PAIR: also the row's pair energy (the edge-force path, whose
 // edge sweep keeps no per-row energy). Without it the window holds the density tables only, so
 // two blocks fit on a CU; the force sweep then sums the pair energy.
-template <typename S, bool HALF, bool PAIR, int G>
-__global__ __launch_bounds__(kRowBlock) void k_eam_density_inc(EamArgs<S> m, TwoSided t,
-                                                               S *__restrict__ rho_part,
-                                                               S *__restrict__ epair)
+template <typename S, bool HALF, bool PAIR, int FILTER, int G>
+__global__ __launch_bounds__(kRowBlock) LK_EIGHT_WAVES
+void k_eam_density_inc(EamArgs<S> m, TwoSided t, S *__restrict__ rho_part, S *__restrict__ epair)
 {
   constexpr int kLds = PAIR ? kIncLds : kIncDensLds;
   constexpr int APB = kRowBlock / G;  // atoms per block
@@ -854,17 +940,17 @@ __global__ __launch_bounds__(kRowBlock) void k_eam_density_inc(EamArgs<S> m, Two
       const BandRow<S> br = band_row(t, xa, m.cutsq);
       const int za = clamp_species(static_cast<int>(xa.w), m.n_el);
       const int b = inc_off(t.loc, t.part, a);
-      const int L = HALF ? inc_off(t.loc, t.part, a + 1) - b : inc_len(t, a, b);  // half: no folds
+      const int L = t.len[a];
       // Two entries per lane at a time (k and k + G): both entries load together, then both
       // records, so a pair of entries costs two memory round trips; a skipped or missing entry
       // gathers the row's own record.
-      auto dens = [&](uint32_t v, int q, const Atom4<S> &xo) {
+      auto dens = [&](uint32_t v, const Atom4<S> &xo) {
         const bool in = (v >> 31) != 0;
         if (!HALF && in) return;  // plain: density and pair energy stay on the sender
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 < m.cutsq)) return;
-        if (!slot_kept(t, q, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
         const S rinv = rsqrt_nr(r2);
         const S rr = r2 * rinv;
         const Locator<S> L2 = locate_mul(rr, m.inv_dr, m.nr);
@@ -891,8 +977,8 @@ __global__ __launch_bounds__(kRowBlock) void k_eam_density_inc(EamArgs<S> m, Two
         const bool s1 = !HALF && (v1 >> 31) != 0, s2 = !two || (!HALF && (v2 >> 31) != 0);
         const Atom4<S> x1 = m.atoms[s1 ? a : static_cast<int>(v1 & kIncAtom)];
         const Atom4<S> x2 = m.atoms[s2 ? a : static_cast<int>(v2 & kIncAtom)];
-        dens(v1, q1, x1);
-        if (two) dens(v2, q2, x2);
+        dens(v1, x1);
+        if (two) dens(v2, x2);
       }
     }
     rho = group_sum<G>(rho);
@@ -1008,7 +1094,7 @@ __device__ __forceinline__ void store_block_partials(double *partials, int blk, 
 // Force sweep (eam.py:336-409 closed form; export.py:197-204 autodiff convention), and the pair
 // energy of the counted rows (eam.py:300-307) from the phi it evaluates anyway: on the sender,
 // both halves in the half scheme, half per directed edge in the plain one.
-template <typename S, bool HALF, bool VIRIAL, bool BITS, int G>
+template <typename S, bool HALF, bool VIRIAL, int FILTER, int G>
 __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const TwoSided &t,
                                                    LdsEntry<S> *lds, int lds_entries)
 {
@@ -1035,20 +1121,18 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
       const int za = clamp_species(static_cast<int>(xa.w), m.n_el);
       const S fpa = m.fp[a];
       const int b = inc_off(t.loc, t.part, a);
-      const int L = HALF ? inc_off(t.loc, t.part, a + 1) - b : inc_len(t, a, b);  // half: no folds
+      const int L = t.len[a];
       // The gathers of an entry: its neighbour's record and F' (the row's own when the entry
       // is skipped, so no branch surrounds a load).
       struct Gathered {
         uint32_t v;
-        int q;  // the entry's index (its slot's bit address is read only near the cutoff)
         bool skip;
         Atom4<S> xo;
         S fpo;
       };
-      auto gather = [&](uint32_t v, int q, bool present) -> Gathered {
+      auto gather = [&](uint32_t v, bool present) -> Gathered {
         Gathered e;
         e.v = v;
-        e.q = q;
         const bool in = (v >> 31) != 0;
         const int o = static_cast<int>(v & kIncAtom);
         // plain: an uncounted sender gives no gradient; a folded pair counts each counted end
@@ -1071,7 +1155,7 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 < m.cutsq)) return;
-        if (BITS && !slot_kept(t, e.q, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
         const S rinv = rsqrt_nr(r2);
         const S rr = r2 * rinv;
         const Locator<S> L2 = locate_mul(rr, m.inv_dr, m.nr);
@@ -1149,7 +1233,7 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
       if constexpr (sizeof(S) == 8) {
         IncCursor<G> cur(t, b, L, gl);
         for (int k = gl; k < L; k += G) {
-          const Gathered e = gather(cur.v, cur.q, true);
+          const Gathered e = gather(cur.v, true);
           cur.advance(t, k);
           edge(e);
         }
@@ -1159,8 +1243,8 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
         uint32_t v1 = static_cast<uint32_t>(t.inc[q1]);
         uint32_t v2 = static_cast<uint32_t>(t.inc[q2]);
         for (int k = gl; k < L; k += 2 * G) {
-          const Gathered e1 = gather(v1, q1, true);
-          const Gathered e2 = gather(v2, q2, k + G < L);
+          const Gathered e1 = gather(v1, true);
+          const Gathered e2 = gather(v2, k + G < L);
           asm volatile("" ::: "memory");  // keep the next entries' loads behind the gathers
           q1 = min(b + k + 2 * G, last);
           q2 = min(b + k + 3 * G, last);
@@ -1191,22 +1275,22 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
 }
 
 // One block per CU: the 120 KB table window (all of a 2000-node r-grid of two elements).
-template <typename S, bool HALF, bool VIRIAL, bool BITS, int G>
+template <typename S, bool HALF, bool VIRIAL, int FILTER, int G>
 __global__ __launch_bounds__(kRowBlock) void k_eam_force_inc(EamArgs<S> m, TwoSided t)
 {
   __shared__ LdsEntry<S> lds[kIncLds];
-  eam_force_inc_rows<S, HALF, VIRIAL, BITS, G>(m, t, lds, kIncLds);
+  eam_force_inc_rows<S, HALF, VIRIAL, FILTER, G>(m, t, lds, kIncLds);
 }
 
 // Two blocks per CU (eight waves per SIMD) with the 64 KB window: twice the gathers in flight for
 // more lookups below the window (L2-resident). The fp32 sweep fits 64 VGPRs without spills
 // (C4 force sweep 814 -> 748 us); the fp64 one would spill.
-template <typename S, bool HALF, bool VIRIAL, bool BITS, int G>
+template <typename S, bool HALF, bool VIRIAL, int FILTER, int G>
 __global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(8))) LK_EIGHT_WAVES
 void k_eam_force_inc_2b(EamArgs<S> m, TwoSided t)
 {
   __shared__ LdsEntry<S> lds[kIncDensLds];
-  eam_force_inc_rows<S, HALF, VIRIAL, BITS, G>(m, t, lds, kIncDensLds);
+  eam_force_inc_rows<S, HALF, VIRIAL, FILTER, G>(m, t, lds, kIncDensLds);
 }
 
 template <typename S>
@@ -1224,7 +1308,7 @@ struct LjModel {
 
 // LJ 12-6 plain (examples/export_model.py:16-50): e per edge on the sender row, g = 2 de/d(r^2) d
 // (times edge_energy_scale) to the sender and minus it to the receiver.
-template <typename S, bool VIRIAL, int G>
+template <typename S, bool VIRIAL, int FILTER, int G>
 __global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(8))) LK_EIGHT_WAVES
 void k_lj_inc(LjModel<S> m, TwoSided t)
 {
@@ -1244,7 +1328,7 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
       const Atom4<S> xa = m.atoms[a];
       const BandRow<S> br = band_row(t, xa, m.cutsq);
       const int b = inc_off(t.loc, t.part, a);
-      const int L = inc_len(t, a, b);
+      const int L = t.len[a];
       // counted ends of an entry: its sender's row, or both rows of a folded pair (the pair
       // force on a is the same from either directed edge)
       auto ends = [&](uint32_t v) -> int {
@@ -1252,12 +1336,12 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
         const int co = static_cast<int>(v & kIncAtom) < erows ? 1 : 0;
         return (in ? 0 : (a < erows ? 1 : 0)) + ((in || (v & kIncPaired)) ? co : 0);
       };
-      auto pair = [&](uint32_t v, int q, int w, const Atom4<S> &xo) {
+      auto pair = [&](uint32_t v, int w, const Atom4<S> &xo) {
         if (w == 0) return;
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 > tiny && r2 < m.cutsq)) return;  // export_model.py:22
-        if (!slot_kept(t, q, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
         const S inv_r2 = m.sigsq / r2;
         const S inv_r6 = inv_r2 * inv_r2 * inv_r2;
         if (!(v >> 31)) en += m.edge_scale * (m.four_eps * (inv_r6 * inv_r6 - inv_r6));
@@ -1277,8 +1361,8 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
         const int w1 = ends(v1), w2 = two ? ends(v2) : 0;
         const Atom4<S> x1 = m.atoms[w1 ? static_cast<int>(v1 & kIncAtom) : a];
         const Atom4<S> x2 = m.atoms[w2 ? static_cast<int>(v2 & kIncAtom) : a];
-        pair(v1, q1, w1, x1);
-        pair(v2, q2, w2, x2);
+        pair(v1, w1, x1);
+        pair(v2, w2, x2);
       }
     }
     en = group_sum<G>(en);
@@ -1327,8 +1411,8 @@ static hipError_t build_incidence(Handle &h, hipStream_t s, int nall)
   const int egrid = grid_for(h, h.contract.max_edges, 256, 16);
   {
     StageTimer timer(h, s, "inc_count");
-    // the counts start from zero whatever the previous build left (a list-built build keeps
-    // out-counts in deg until its sort clears them)
+    // the counts start from zero whatever the previous build left (a list-built one keeps the
+    // rows' slot counts there)
     const long n = static_cast<long>(h.contract.max_atoms) + 1;
     hipLaunchKernelGGL(k_clear_int, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s,
                        h.d_deg, n);
@@ -1353,11 +1437,7 @@ static hipError_t build_incidence(Handle &h, hipStream_t s, int nall)
   return hipGetLastError();
 }
 
-// Lists of at most this many slots sort all of them (the unused tail padded) instead of reading
-// the kept count back: the read back would stall the stream for more than the padding costs.
-constexpr long kIncSortExact = 1L << 22;
-
-static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, int nall, bool fold)
+static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
 {
   ListArgs L;
   L.ilist = h.list_ilist;
@@ -1368,157 +1448,89 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, int nall, 
   L.maxneighs = h.list_maxneighs;
   L.max_atoms = h.contract.max_atoms;
   L.half_filter = h.list_half_filter;
-  L.pitch = h.contract.max_atoms;
-  L.deg = h.d_deg;
+  L.out_n = h.d_deg;
+  L.row_of = h.d_row_of;
   L.loc = h.d_inc_loc;
   L.part = h.d_inc_part;
-  L.tmp = h.d_inc_tmp;
-  L.inc = h.d_inc;
   L.len = h.d_inc_len;
-  L.fold = fold ? 1 : 0;
-  L.inc_bit = h.d_inc_bit;
-  const int rows = L.rows;
-  const int atoms = h.contract.max_atoms;
-  // at most one in-entry per list slot (ensure_incidence keeps rows * maxneighs within int)
-  const long slots_max = static_cast<long>(rows) * L.maxneighs;
-  // keys are atoms below max_atoms; the pad key (all ones in key_bits) sorts above them all
-  int key_bits = 1;
-  while ((1L << key_bits) <= atoms) ++key_bits;
-  const uint32_t pad = static_cast<uint32_t>((1L << key_bits) - 1);
-  hipError_t e = hipSuccess;
-  if (slots_max > h.sort_cap || rows + 1L > h.sort_rows_cap || !h.d_sort_pre) {
-    // the working arrays grow (rarely) for a larger list; a previous build may still use them
-    size_t b_scan_rows = 0, b_scan_atoms = 0, b_sort = 0;
-    const int cap = static_cast<int>(slots_max > 0 ? slots_max : 1);
-    e = hipcub::DeviceScan::ExclusiveSum(nullptr, b_scan_rows, static_cast<int *>(nullptr),
-                                         static_cast<int *>(nullptr), rows + 1, s);
-    if (e == hipSuccess)
-      e = hipcub::DeviceScan::ExclusiveSum(nullptr, b_scan_atoms, static_cast<int *>(nullptr),
-                                           static_cast<int *>(nullptr), atoms + 2, s);
-    if (e == hipSuccess)
-      e = rocprim::radix_sort_pairs<IncSortConfig>(nullptr, b_sort, static_cast<uint32_t *>(nullptr),
-                                                   static_cast<uint32_t *>(nullptr),
-                                                   static_cast<uint32_t *>(nullptr),
-                                                   static_cast<uint32_t *>(nullptr), cap, 0u,
-                                                   static_cast<unsigned>(key_bits), s);
-    if (e != hipSuccess) return e;
-    const size_t tmp = std::max(b_sort, std::max(b_scan_rows, b_scan_atoms));
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
-    for (void *q : {static_cast<void *>(h.d_sort_keys), static_cast<void *>(h.d_sort_vals),
-                    static_cast<void *>(h.d_sort_rows), static_cast<void *>(h.d_sort_pre),
-                    h.d_sort_tmp})
-      if (q) (void)hipFree(q);
-    h.d_sort_keys = nullptr;
-    h.d_sort_vals = nullptr;
-    h.d_sort_rows = nullptr;
-    h.d_sort_pre = nullptr;
-    h.d_sort_tmp = nullptr;
-    h.sort_cap = h.sort_rows_cap = 0;
-    h.sort_tmp_bytes = 0;
-    if ((e = hipMalloc(&h.d_sort_keys, 2 * static_cast<size_t>(cap) * sizeof(uint32_t))) != hipSuccess) return e;
-    if ((e = hipMalloc(&h.d_sort_vals, 2 * static_cast<size_t>(cap) * sizeof(uint32_t))) != hipSuccess) return e;
-    if ((e = hipMalloc(&h.d_sort_rows, 2 * (static_cast<size_t>(rows) + 1) * sizeof(int))) != hipSuccess) return e;
-    if ((e = hipMalloc(&h.d_sort_pre, (static_cast<size_t>(atoms) + 2) * sizeof(int))) != hipSuccess) return e;
-    if ((e = hipMalloc(&h.d_sort_tmp, tmp > 0 ? tmp : 1)) != hipSuccess) return e;
-    h.sort_cap = cap;
-    h.sort_rows_cap = rows + 1L;
-    h.sort_tmp_bytes = tmp;
+  L.inc = h.d_inc;
+  const int atoms = L.max_atoms;
+  // Atoms per bin: 64, or fewer where the out-entries of that many rows and their in-entries (with
+  // a fold, hash tables four fifths full at the list's width) would take more than 62 KB of LDS
+  // (two blocks or more share a CU). Rows past 1,700 slots go through memory.
+  constexpr long kPool = 62 * 1024;
+  const long per = fold ? (L.maxneighs * 5L / 4 + 7) / 4 * 4 : (L.maxneighs + 7L) / 4 * 4;
+  const int pitch = L.maxneighs | 1;
+  L.bin_log = kBinLog;
+  while (L.bin_log > 2 && 4 * (per + pitch) << L.bin_log > kPool) --L.bin_log;
+  const bool staged = 4 * (per + pitch) << L.bin_log <= kPool;
+  const int per_atom = staged ? static_cast<int>(per) : 0;
+  const size_t lds = staged ? static_cast<size_t>(4 * (per + pitch)) << L.bin_log : 0;
+  Bins B;
+  B.n = (atoms + (1 << L.bin_log) - 1) >> L.bin_log;
+  if (4L * B.n + 2 > h.bins_cap) {  // rarely: rows that need smaller bins; a build may be running
+    if (hipError_t e = hipDeviceSynchronize(); e != hipSuccess) return e;
+    if (h.d_bins) (void)hipFree(h.d_bins);
+    h.d_bins = nullptr;
+    h.bins_cap = 0;
+    if (hipError_t e = hipMalloc(&h.d_bins, (4L * B.n + 2) * sizeof(int)); e != hipSuccess) return e;
+    h.bins_cap = 4L * B.n + 2;
   }
-  uint32_t *keys_in = h.d_sort_keys, *keys_out = h.d_sort_keys + h.sort_cap;
-  uint32_t *vals_in = h.d_sort_vals, *vals_out = h.d_sort_vals + h.sort_cap;
-  const int ntiles = (rows + kWave - 1) / kWave;
-  int *tilecnt = h.d_sort_rows, *tileoff = h.d_sort_rows + (ntiles + 1);
-  int kept = 0;
+  B.next = h.d_bins;
+  B.out = B.next + B.n;
+  B.off = B.out + B.n;
+  B.loff = B.off + B.n + 1;
+  const dim3 row_grid((L.rows + kBinTiles * kWave - 1) / (kBinTiles * kWave));
+  constexpr int kRowThreads = kBinTiles * kBinW * kWave;
   {
     StageTimer timer(h, s, "inc_count");
-    const long n = static_cast<long>(atoms) + 2;  // deg holds max_atoms + 2 counts
-    hipLaunchKernelGGL(k_clear_int, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s,
-                       h.d_deg, n);
-    const int chunks = (atoms + 1 + kScanChunk - 1) / kScanChunk;
-    hipLaunchKernelGGL(k_clear_int, dim3((chunks + 255) / 256), dim3(256), 0, s, h.d_inc_part,
-                       static_cast<long>(chunks));
-    hipLaunchKernelGGL(k_inc_tiles_count, dim3((ntiles + 1 + 3) / 4), dim3(256), 0, s, L, ntiles,
-                       tilecnt);
-    size_t bytes = h.sort_tmp_bytes;
-    if ((e = hipcub::DeviceScan::ExclusiveSum(h.d_sort_tmp, bytes, tilecnt, tileoff, ntiles + 1,
-                                              s)) != hipSuccess)
-      return e;
-    if (slots_max > kIncSortExact) {
-      // a large list: the in-entry count sizes the sort (one read back per list)
-      if ((e = hipMemcpyAsync(&kept, tileoff + ntiles, sizeof(int), hipMemcpyDeviceToHost, s)) !=
-          hipSuccess)
-        return e;
-      if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-    } else {
-      // a small one: the sort takes every slot, its unused tail padded, and nothing waits
-      kept = static_cast<int>(slots_max);
+    hipLaunchKernelGGL(k_inc_clear, dim3((atoms + 255) / 256), dim3(256), 0, s, L, B);
+    if (L.rows > 0)
+      hipLaunchKernelGGL((k_inc_bins<false, uint32_t>), row_grid, dim3(kRowThreads), 0, s, L, B,
+                         static_cast<uint32_t *>(nullptr));
+    hipLaunchKernelGGL(k_inc_bin_scan, dim3(1), dim3(kScanThreads), 0, s, B);
+  }
+  auto finish = [&](auto *tmp) {
+    using E = std::remove_pointer_t<decltype(tmp)>;
+    if (L.rows > 0) {
+      StageTimer timer(h, s, "inc_fill");
+      hipLaunchKernelGGL((k_inc_bins<true, E>), row_grid, dim3(kRowThreads), 0, s, L, B, tmp);
     }
-  }
-  if (ntiles > 0) {
-    StageTimer timer(h, s, "inc_fill");
-    hipLaunchKernelGGL(k_inc_tiles_emit, dim3((ntiles + 3) / 4), dim3(256), 0, s, L, ntiles,
-                       tileoff, keys_in, vals_in);
-  }
-  if (kept > 0 && slots_max <= kIncSortExact)
-    hipLaunchKernelGGL(k_inc_pad_keys, dim3((kept + 255) / 256), dim3(256), 0, s, keys_in,
-                       tileoff + ntiles, kept, pad);
-  if (kept > 0) {
-    StageTimer timer(h, s, "inc_sort");
-    size_t bytes = h.sort_tmp_bytes;
-    if ((e = rocprim::radix_sort_pairs<IncSortConfig>(h.d_sort_tmp, bytes, keys_in, keys_out,
-                                                      vals_in, vals_out, kept, 0u,
-                                                      static_cast<unsigned>(key_bits), s)) !=
-        hipSuccess)
-      return e;
-  }
-  {
-    StageTimer timer(h, s, "inc_scan");
-    // pre[a] = out-entries of the atoms below a (deg holds each atom's out-entries; deg[atoms]
-    // and deg[atoms + 1] are zero)
-    size_t bytes = h.sort_tmp_bytes;
-    if ((e = hipcub::DeviceScan::ExclusiveSum(h.d_sort_tmp, bytes, h.d_deg, h.d_sort_pre,
-                                              atoms + 2, s)) != hipSuccess)
-      return e;
-    hipLaunchKernelGGL(k_inc_atoms_loc, dim3((atoms + 1 + 255) / 256), dim3(256), 0, s, keys_out,
-                       kept, h.d_sort_pre, atoms, h.d_inc_loc);
-  }
-  {
     StageTimer timer(h, s, "inc_place");
-    // out-entries staged in LDS per tile when the slot numbers fit a byte, else row by row. Rows
-    // padded to the longest (pitch), or runs packed at 5/4 of the mean run per row (the list
-    // entries read back for a large list; the longest row at least) when that staging is no
-    // larger: ragged rows. (C4's half list, 48 of 105 slots on average: place 978 -> 785 us a
-    // rebuild with the runs; C5's even rows lost 22 us with them.) Either staging stays within
-    // 64 KB of dynamic LDS; a larger one goes row by row.
-    const int pitch = L.maxneighs | 1;
-    const size_t lds_rows = static_cast<size_t>(kWave) * pitch * (sizeof(int) + 1);
-    const long mean_run = kept > 0 && rows > 0 ? (static_cast<long>(kept) + rows - 1) / rows
-                                               : L.maxneighs;
-    const int cap = static_cast<int>(std::max<long>(
-        L.maxneighs, std::min<long>(static_cast<long>(kWave) * L.maxneighs,
-                                    kWave * ((mean_run * 5 + 3) / 4))));
-    const size_t lds_runs = static_cast<size_t>(cap) * (sizeof(int) + 2) + 2 * kWave * sizeof(int);
-    if (L.maxneighs <= 255 && lds_runs <= lds_rows && lds_runs <= 65536) {
-      if (ntiles > 0)
-        hipLaunchKernelGGL(k_inc_tiles_place_runs, dim3(ntiles), dim3(kWave), lds_runs, s, L,
-                           ntiles, cap);
-    } else if (L.maxneighs <= 255 && lds_rows <= 65536) {
-      if (ntiles > 0)
-        hipLaunchKernelGGL(k_inc_tiles_place, dim3(ntiles), dim3(kWave), lds_rows, s, L, ntiles,
-                           pitch);
-    } else {
-      hipLaunchKernelGGL(k_inc_rows_place, dim3((rows + 255) / 256), dim3(256), 0, s, L);
-    }
-    if (kept > 0)
-      hipLaunchKernelGGL(k_inc_sorted_place, dim3((kept + 255) / 256), dim3(256), 0, s, L,
-                         keys_out, vals_out, kept, h.d_sort_pre);
-  }
-  if (L.fold && nall > 0) {
-    StageTimer timer(h, s, "inc_fold");
-    hipLaunchKernelGGL(k_inc_list_fold_sorted, dim3((nall + 256 / kFoldLanes - 1) / (256 / kFoldLanes)),
-                       dim3(256), 0, s, L, nall);
-  }
+    if (fold)
+      hipLaunchKernelGGL((k_inc_lists<E, true>), dim3(B.n), dim3(kListThreads), lds, s, L, B, tmp,
+                         per_atom, pitch);
+    else
+      hipLaunchKernelGGL((k_inc_lists<E, false>), dim3(B.n), dim3(kListThreads), lds, s, L, B, tmp,
+                         per_atom, pitch);
+  };
+  // d_inc_tmp holds two words per list slot (ensure_incidence)
+  if (atoms <= kBinAtoms32)
+    finish(h.d_inc_tmp);
+  else
+    finish(reinterpret_cast<uint64_t *>(h.d_inc_tmp));
   return hipGetLastError();
+}
+
+// The sweeps' filter: none for lists built from packed edges or from a matrix, whose slots the
+// model masks itself.
+static int sweep_filter(const Handle &h, bool from_list, const FusedPack &pack)
+{
+  if (!from_list || !h.list_bits_filter) return kAllKept;
+  return pack.state ? kFromX : kFromBits;
+}
+
+// Calls f with `filter` as a constant. Float64 sweeps decide every entry from its own r2, so one
+// filtering form serves both.
+template <typename S, class F>
+static void with_filter(int filter, F &&f)
+{
+  if (filter == kAllKept)
+    f(std::integral_constant<int, kAllKept>{});
+  else if (sizeof(S) == 8 || filter == kFromX)
+    f(std::integral_constant<int, kFromX>{});
+  else if constexpr (sizeof(S) == 4)
+    f(std::integral_constant<int, kFromBits>{});
 }
 
 static TwoSided two_sided_args(Handle &h, int nlocal, int nghost, const double *x)
@@ -1527,7 +1539,7 @@ static TwoSided two_sided_args(Handle &h, int nlocal, int nghost, const double *
   t.loc = h.d_inc_loc;
   t.part = h.d_inc_part;
   t.inc = h.d_inc;
-  t.len = h.inc_key.fold ? h.d_inc_len : nullptr;  // set by the list build that folded
+  t.len = h.d_inc_len;
   t.nall = nlocal + nghost;
   t.nlocal = nlocal;
   t.nadd = h.contract.newton_pair ? t.nall : nlocal;
@@ -1537,8 +1549,12 @@ static TwoSided two_sided_args(Handle &h, int nlocal, int nghost, const double *
   t.ghost_off = nghost > 0 ? h.d_ghost_off : nullptr;
   t.ghost_list = h.d_ghost_list;
   t.nblk = (t.nall + kRowAtoms - 1) / kRowAtoms;
-  t.inc_bit = nullptr;
   t.bits = h.d_bits;
+  t.row_of = h.d_row_of;
+  t.out_n = h.d_deg;
+  t.neighbors = h.inc_key.neighbors;
+  t.stride = h.inc_key.stride;
+  t.max_atoms = h.contract.max_atoms;
   t.cutsq_pack = h.contract.cutoff * h.contract.cutoff;
   t.cutsq_lo = static_cast<float>(t.cutsq_pack);
   t.cutsq_hi = t.cutsq_lo;
@@ -1568,7 +1584,7 @@ static hipError_t eam_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost
   EamArgs<S> m = eam_args<S>(h, nlocal, scale, f);
   TwoSided t = two_sided_args(h, nlocal, nghost, x);
   use_pack(t, pack);
-  if (from_list && h.list_bits_filter) t.inc_bit = h.d_inc_bit;
+  const int filter = sweep_filter(h, from_list, pack);
   m.flags = flags;
   // Split passes exchange the handle's rho rows: the density sweep writes its partials there and
   // the embedding reads them back completed (every row, ghosts included, holding its atom's
@@ -1584,8 +1600,11 @@ static hipError_t eam_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost
   const int grid = grid_for(h, nsb, 1, 1);
   if (t.nblk > 0 && phase != kPhaseForce) {
     StageTimer timer(h, s, "eam_density");
-    hipLaunchKernelGGL((k_eam_density_inc<S, HALF, false, G>), dim3(grid_for(h, nsb, 1, 2)),
-                       dim3(kRowBlock), 0, s, m, t, rho_part, static_cast<S *>(nullptr));
+    with_filter<S>(filter, [&](auto F) {
+      hipLaunchKernelGGL((k_eam_density_inc<S, HALF, false, F.value, G>),
+                         dim3(grid_for(h, nsb, 1, 2)), dim3(kRowBlock), 0, s, m, t, rho_part,
+                         static_cast<S *>(nullptr));
+    });
   }
   if (phase == kPhaseDensity) return hipGetLastError();
   if (t.nblk > 0) {
@@ -1599,27 +1618,20 @@ static hipError_t eam_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost
   }
   // one launch even with no rows: its last block writes the step result
   StageTimer timer(h, s, "eam_force");
-  const bool vir = (flags & LK_VIRIAL) != 0;
-  if constexpr (kForceTwoBlocks<S>) {
-    const int grid2 = grid_for(h, nsb, 1, 2);
-    if (vir && t.inc_bit)
-      hipLaunchKernelGGL((k_eam_force_inc_2b<S, HALF, true, true, G>), dim3(grid2), dim3(kRowBlock), 0, s, m, t);
-    else if (vir)
-      hipLaunchKernelGGL((k_eam_force_inc_2b<S, HALF, true, false, G>), dim3(grid2), dim3(kRowBlock), 0, s, m, t);
-    else if (t.inc_bit)
-      hipLaunchKernelGGL((k_eam_force_inc_2b<S, HALF, false, true, G>), dim3(grid2), dim3(kRowBlock), 0, s, m, t);
+  with_filter<S>(filter, [&](auto F) {
+    auto launch = [&](auto virial) {
+      if constexpr (kForceTwoBlocks<S>)
+        hipLaunchKernelGGL((k_eam_force_inc_2b<S, HALF, virial.value, F.value, G>),
+                           dim3(grid_for(h, nsb, 1, 2)), dim3(kRowBlock), 0, s, m, t);
+      else
+        hipLaunchKernelGGL((k_eam_force_inc<S, HALF, virial.value, F.value, G>), dim3(grid),
+                           dim3(kRowBlock), 0, s, m, t);
+    };
+    if (flags & LK_VIRIAL)
+      launch(std::true_type{});
     else
-      hipLaunchKernelGGL((k_eam_force_inc_2b<S, HALF, false, false, G>), dim3(grid2), dim3(kRowBlock), 0, s, m, t);
-  } else {
-    if (vir && t.inc_bit)
-      hipLaunchKernelGGL((k_eam_force_inc<S, HALF, true, true, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
-    else if (vir)
-      hipLaunchKernelGGL((k_eam_force_inc<S, HALF, true, false, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
-    else if (t.inc_bit)
-      hipLaunchKernelGGL((k_eam_force_inc<S, HALF, false, true, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
-    else
-      hipLaunchKernelGGL((k_eam_force_inc<S, HALF, false, false, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
-  }
+      launch(std::false_type{});
+  });
   return hipGetLastError();
 }
 
@@ -1643,15 +1655,17 @@ static hipError_t lj_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost,
   m.mirror = h.d_host_result;
   TwoSided t = two_sided_args(h, nlocal, nghost, x);
   use_pack(t, pack);
-  if (from_list && h.list_bits_filter) t.inc_bit = h.d_inc_bit;
+  const int filter = sweep_filter(h, from_list, pack);
   constexpr int G = kLanesPerAtom<S>;
   const int nsb = t.nall > 0 ? (t.nall + kRowBlock / G - 1) / (kRowBlock / G) : 1;
   const int grid = grid_for(h, nsb, 1, 2);
   StageTimer timer(h, s, "lj_rows");
-  if (flags & LK_VIRIAL)
-    hipLaunchKernelGGL((k_lj_inc<S, true, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
-  else
-    hipLaunchKernelGGL((k_lj_inc<S, false, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
+  with_filter<S>(filter, [&](auto F) {
+    if (flags & LK_VIRIAL)
+      hipLaunchKernelGGL((k_lj_inc<S, true, F.value, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
+    else
+      hipLaunchKernelGGL((k_lj_inc<S, false, F.value, G>), dim3(grid), dim3(kRowBlock), 0, s, m, t);
+  });
   return hipGetLastError();
 }
 
@@ -1917,15 +1931,16 @@ static hipError_t eam_edge_force(Handle &h, hipStream_t s, int nlocal, int nghos
 {
   EamArgs<S> m = eam_args<S>(h, nlocal, scale, f);
   TwoSided t = two_sided_args(h, nlocal, nghost, x);
-  if (from_list && h.list_bits_filter) t.inc_bit = h.d_inc_bit;
   m.flags = flags;
   S *rho_part = static_cast<S *>(h.d_rho_part);
   S *epair = static_cast<S *>(h.d_epair);
   if (t.nblk > 0) {
     StageTimer timer(h, s, "eam_density");
-    hipLaunchKernelGGL((k_eam_density_inc<S, true, true, 16>),
-                       dim3(grid_for(h, (t.nall + kRowBlock / 16 - 1) / (kRowBlock / 16), 1, 1)),
-                       dim3(kRowBlock), 0, s, m, t, rho_part, epair);
+    with_filter<S>(sweep_filter(h, from_list, FusedPack{}), [&](auto F) {
+      hipLaunchKernelGGL((k_eam_density_inc<S, true, true, F.value, 16>),
+                         dim3(grid_for(h, (t.nall + kRowBlock / 16 - 1) / (kRowBlock / 16), 1, 1)),
+                         dim3(kRowBlock), 0, s, m, t, rho_part, epair);
+    });
   }
   if (t.nblk > 0) {
     StageTimer timer(h, s, "eam_embed");
@@ -1991,7 +2006,7 @@ hipError_t launch_edge_force(Handle &h, hipStream_t s, int nlocal, int nghost, i
     key.half_filter = h.list_half_filter;
     key.fold = 0;  // the edge-force sweeps walk whole lists
     if (h.list_epoch < 0 || !(key == h.inc_key)) {
-      e = build_incidence_from_list(h, s, nlocal + nghost, false);
+      e = build_incidence_from_list(h, s, false);
       h.inc_key = key;
     }
   } else {
@@ -2022,7 +2037,7 @@ hipError_t launch_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost, in
     key.half_filter = h.list_half_filter;
     key.fold = h.accum == LK_ACCUM_PLAIN ? 1 : 0;
     if (h.list_epoch < 0 || !(key == h.inc_key)) {
-      e = build_incidence_from_list(h, s, nlocal + nghost, key.fold != 0);
+      e = build_incidence_from_list(h, s, key.fold != 0);
       h.inc_key = key;
     }
   } else {
