@@ -112,7 +112,7 @@ static void set_pack_cutoff(StepPack &p, double cutoff)
     p.cutsq_hi = std::nextafter(p.cutsq_hi, std::numeric_limits<float>::infinity());
 }
 
-constexpr int kStepW = 4, kStepTPB = 4;
+constexpr int kStepWaves = 16;    // waves per block: kStepWaves / W tiles
 constexpr int kStepLds = 3584;     // table window entries: 56 KB (two blocks per CU)
 constexpr int kStepMaxWords = 8;   // validity words kept in LDS for the write (256 list slots)
 
@@ -132,11 +132,11 @@ static int step_pack_grid(int ngroups, int num_cus)
   return ((ngroups + kXcds - 1) / kXcds) * kXcds;
 }
 
-template <typename S, bool EAM, bool MATRIX>
-__global__ __launch_bounds__(kStepW * kStepTPB * 64) __attribute__((amdgpu_waves_per_eu(8))) LK_EIGHT_WAVES
+template <typename S, bool EAM, bool MATRIX, int W>
+__global__ __launch_bounds__(kStepWaves * kWave) __attribute__((amdgpu_waves_per_eu(8))) LK_EIGHT_WAVES
 void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
 {
-  constexpr int W = kStepW, TPB = kStepTPB;
+  constexpr int TPB = kStepWaves / W;
   __shared__ LdsEntry<S> lds[EAM ? kStepLds : 1];
   __shared__ int cpart[TPB][W][kWave];
   __shared__ S rpart[TPB][W][kWave];
@@ -182,7 +182,7 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
       xi0 = p.x[3L * i + 0];
       xi1 = p.x[3L * i + 1];
       xi2 = p.x[3L * i + 2];
-      if constexpr (sizeof(S) == 4 && !EAM) xa = a.atoms[i];
+      if constexpr (sizeof(S) == 4) xa = a.atoms[i];
     }
     const float sa = fabsf(xa.x) + fabsf(xa.y) + fabsf(xa.z);
     const int nn_max = wave_max_int(nn);
@@ -197,72 +197,47 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
     auto slot_entry = [&](int jj) -> int {
       return p.neighbors[jj < nn ? static_cast<long>(jj) * p.stride + i : 0L];
     };
-    // One list slot of this lane's row (entry: its list entry): the filter chain, and the density
-    // of a kept pair (the model kernels).
+    // One list slot of this lane's row (entry: its list entry) in the float64 model kernels: the
+    // filter chain, and the density of a kept pair.
     auto visit = [&](int jj, int entry) -> bool {
-      const int j = entry & kNeighMask;
-      if (!(jj < nn && j < p.max_atoms)) return false;
-      double rsq;
-      double xj0, xj1, xj2;
-      int zj = 0;
-      if constexpr (sizeof(S) == 8) {
-        // float64 records hold the engine's x exactly: one 32-byte gather (two 16-byte loads)
-        // brings x and species. The empty asm takes the species where it arrives, so the
-        // compiler cannot defer it into an 8-byte gather of its own behind the filter.
+      if constexpr (EAM && sizeof(S) == 8) {
+        const int j = entry & kNeighMask;
+        if (!(jj < nn && j < p.max_atoms)) return false;
+        // one 32-byte gather (two 16-byte loads) brings x and species. The empty asm takes the
+        // species where it arrives, so the compiler cannot defer it into an 8-byte gather of its
+        // own behind the filter.
         const Atom4<double> rj = reinterpret_cast<const Atom4<double> *>(a.atoms)[j];
         asm volatile("" ::"v"(rj.w));
-        xj0 = rj.x;
-        xj1 = rj.y;
-        xj2 = rj.z;
-        zj = static_cast<int>(rj.w);
-      } else {
-        xj0 = p.x[3L * j + 0];
-        xj1 = p.x[3L * j + 1];
-        xj2 = p.x[3L * j + 2];
-        if constexpr (EAM) zj = p.type[j] - 1;
-      }
-      {
+        double rsq;
+        {
 #pragma clang fp contract(off)
-        const double dx = xi0 - xj0, dy = xi1 - xj1, dz = xi2 - xj2;
-        rsq = dx * dx + dy * dy + dz * dz;
-      }
-      if constexpr (!MATRIX) {
-        if (rsq > p.cutsq) return false;  // PackNeighborFunctor keeps rsq <= cutsq (cpp:91)
-      }
-      S r2 = S(0);
-      if constexpr (EAM) {
-        if constexpr (sizeof(S) == 8) {
-          r2 = rsq;  // the model's (x_j - x_i)^2 sum is the same float64 value
+          const double dx = xi0 - rj.x, dy = xi1 - rj.y, dz = xi2 - rj.z;
+          rsq = dx * dx + dy * dy + dz * dz;
+        }
+        if constexpr (MATRIX) {
+          if (!(rsq < a.cutsq)) return false;
         } else {
-#pragma clang fp contract(off)
-          const S dx = static_cast<S>(xj0) - static_cast<S>(xi0);
-          const S dy = static_cast<S>(xj1) - static_cast<S>(xi1);
-          const S dz = static_cast<S>(xj2) - static_cast<S>(xi2);
-          r2 = dx * dx + dy * dy + dz * dz;
+          if (rsq > p.cutsq) return false;  // PackNeighborFunctor keeps rsq <= cutsq (cpp:91)
         }
-      }
-      if constexpr (MATRIX) {
-        if (!(r2 < a.cutsq)) return false;
-      }
-      ++cnt;
-      if constexpr (EAM) {
-        if (MATRIX || r2 < a.cutsq) {  // valid = mask & r_sq < cutoff_sq (eam.py:288)
-          const S rr = r2 * rsqrt_nr(r2);
-          const Locator<S> L = locate_mul(rr, a.inv_dr, a.nr);
-          rho += cvalue(rcoef(win, a, L.node, clamp_species(zj, a.n_el)), L.t);
+        ++cnt;
+        if (MATRIX || rsq < a.cutsq) {  // valid = mask & r_sq < cutoff_sq (eam.py:288)
+          const double rr = rsq * rsqrt_nr(rsq);
+          const Locator<double> L = locate_mul(rr, static_cast<double>(a.inv_dr), a.nr);
+          rho += cvalue(rcoef(win, a, L.node, clamp_species(static_cast<int>(rj.w), a.n_el)), L.t);
         }
+        return true;
       }
-      return true;
+      return false;
     };
-    // Pack-only kernels (no model in the loop, registers to spare) walk the slots jj0,
-    // jj0 + step, ... < jj1 two at a time: both entries are loaded one pair ahead, then both
+    // The float32 and the pack-only kernels walk the slots jj0, jj0 + step, ... < jj1 two at a time: both entries are loaded one pair ahead, then both
     // neighbour records gathered together, so a pair costs one memory round trip. Every load
     // is unconditional (slots past the row read element 0 of the list and the record of atom 0,
     // which exist whenever the loop runs, and are unused), so the compiler counts them exactly
     // and waits for the gathers without waiting for the next pair's entries. The records are
     // this step's (K0 ran before, or the engine's lk_pack_atoms call): float64 ones hold x
-    // exactly; float32 ones decide the filter through pack_keeps_f32 (one 16-byte gather per
-    // slot instead of three 8-byte ones from x).
+    // exactly; float32 ones decide the filter through pack_keeps_f32 and give the model its r^2
+    // and the neighbour's species (one 16-byte gather per slot in place of three 8-byte ones from
+    // x and one from type: 104,284 atoms' matrix 83 -> 57 us, at eight waves per tile).
     auto walk32 = [&](int jj0, int jj1, int step, auto &&kept) {
       auto gather = [&](int jj, int entry) -> Atom4<float> {
         const int j = entry & kNeighMask;
@@ -270,9 +245,27 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
       };
       auto test = [&](int jj, int entry, const Atom4<float> &xo) {
         const int j = entry & kNeighMask;
-        if (jj < nn && j < p.max_atoms && pack_keeps_f32(p, xa, sa, xo, j, xi0, xi1, xi2)) {
-          ++cnt;
-          kept(jj);
+        if (!(jj < nn && j < p.max_atoms)) return;
+        float r2 = 0.0f;
+        if constexpr (EAM) {
+#pragma clang fp contract(off)
+          const float dx = xo.x - xa.x, dy = xo.y - xa.y, dz = xo.z - xa.z;
+          r2 = dx * dx + dy * dy + dz * dz;
+        }
+        if constexpr (MATRIX) {
+          if (!(r2 < a.cutsq)) return;
+        } else {
+          if (!pack_keeps_f32(p, xa, sa, xo, j, xi0, xi1, xi2)) return;
+        }
+        ++cnt;
+        kept(jj);
+        if constexpr (EAM && sizeof(S) == 4) {
+          if (MATRIX || r2 < a.cutsq) {  // valid = mask & r_sq < cutoff_sq (eam.py:288)
+            const float rr = r2 * rsqrt_nr(r2);
+            const Locator<float> L = locate_mul(rr, a.inv_dr, a.nr);
+            rho += cvalue(rcoef(win, a, L.node, clamp_species(static_cast<int>(xo.w), a.n_el)),
+                          L.t);
+          }
         }
       };
       int ea = slot_entry(jj0), eb = slot_entry(jj0 + step);
@@ -332,47 +325,38 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
         }
       }
     };
-    // Rows of fewer than W words (half lists) would leave waves idle under one word per wave:
-    // there each wave takes every W-th slot and ORs its bits into the tile's LDS words, which
-    // the first barrier below completes (the global words are stored after it).
-    const bool strided = nwords < W;
-    if (strided && wave == 0)
-      for (int w = 0; w < nwords; ++w) sbits[sub][w][lane] = 0u;
+    // Each wave takes every W-th slot and ORs its bits into the tile's LDS words, which the first
+    // barrier below completes (the global words are stored after it); rows of more words than
+    // LDS holds go one word per wave at a time.
+        if (lds_bits)
+      for (int w = wave; w < nwords; w += W) sbits[sub][w][lane] = 0u;
     __syncthreads();
-    if (strided) {
-      for (int w = 0; w < nwords; ++w) {
-        uint32_t part = 0;
-        if constexpr (EAM) {
-          for (int k = wave; k < 32; k += W) {
-            const int jj = w * 32 + k;
-            if (jj >= nn_max) break;
-            if (visit(jj, slot_entry(jj))) part |= 1u << k;
-          }
-        } else {
-          walk(w * 32 + wave, min(w * 32 + 32, nn_max), W,
-               [&](int jj) { part |= 1u << (jj & 31); });
-        }
-        if (part) atomicOr(&sbits[sub][w][lane], part);
+    if (lds_bits) {
+      auto mark = [&](int jj) { atomicOr(&sbits[sub][jj >> 5][lane], 1u << (jj & 31)); };
+      if constexpr (EAM && sizeof(S) == 8) {
+        for (int jj = wave; jj < nn_max; jj += W)
+          if (visit(jj, slot_entry(jj))) mark(jj);
+      } else if (wave < nn_max) {
+        walk(wave, nn_max, W, mark);
       }
     } else {
       for (int w = wave; w < nwords; w += W) {
         uint32_t word = 0;
         const int jj0 = w * 32;
         const int jj1 = min(jj0 + 32, nn_max);
-        if constexpr (EAM) {
+        if constexpr (EAM && sizeof(S) == 8) {
           for (int jj = jj0; jj < jj1; ++jj)
             if (visit(jj, slot_entry(jj))) word |= 1u << (jj & 31);
         } else {
           walk(jj0, jj1, 1, [&](int jj) { word |= 1u << (jj & 31); });
         }
         if (row) p.bits[static_cast<long>(w) * p.pitch + ii] = word;
-        if (lds_bits) sbits[sub][w][lane] = word;
       }
     }
     cpart[sub][wave][lane] = cnt;
     if constexpr (EAM) rpart[sub][wave][lane] = rho;
     __syncthreads();
-    if (strided && row)
+    if (lds_bits && row)
       for (int w = wave; w < nwords; w += W)
         p.bits[static_cast<long>(w) * p.pitch + ii] = sbits[sub][w][lane];
     if (wave == 0) {
@@ -496,6 +480,18 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
   }
 }
 
+// The pack alone (two-sided and LJ steps).
+template <typename S>
+static void launch_pack_rows(Handle &h, hipStream_t s, const StepPack &p, const EamArgs<S> &a,
+                             int ntiles)
+{
+  constexpr int W = 8, TPB = kStepWaves / W;
+  const int ngroups = (ntiles + TPB - 1) / TPB;
+  hipLaunchKernelGGL((k_step_pack<S, false, false, W>),
+                     dim3(step_pack_grid<false>(ngroups, h.num_cus)), dim3(kStepWaves * kWave), 0,
+                     s, p, a, ngroups);
+}
+
 // Starts a pack without the atom records (matrix bundles, whose records come from a separate
 // lk_pack_atoms): zeroes the demand count and the ghost-sender flag.
 __global__ void k_clear_state(int *state)
@@ -562,7 +558,6 @@ static hipError_t step_onesided(Handle &h, hipStream_t s, const double *x, const
   p.species_out = nullptr;
   p.records = 0;
   const int ntiles = (num_rows + kWave - 1) / kWave;
-  const int ngroups = ntiles > 0 ? (ntiles + kStepTPB - 1) / kStepTPB : 1;
   // float64 EAM over an engine list: the pack and density over tile lists (lk_tiles.hip)
   bool tiled = false;
   if constexpr (EAM && !MATRIX && sizeof(S) == 8) tiled = tile_step_eligible(h, num_rows, maxneighs);
@@ -594,9 +589,25 @@ static hipError_t step_onesided(Handle &h, hipStream_t s, const double *x, const
   }
   if (ntiles > 0 && !tiled) {
     StageTimer timer(h, s, "step_pack");
-    const int grid = step_pack_grid<EAM>(ngroups, h.num_cus);
-    hipLaunchKernelGGL((k_step_pack<S, EAM, MATRIX>), dim3(grid),
-                       dim3(kStepW * kStepTPB * kWave), 0, s, p, a, ngroups);
+    if constexpr (!EAM) {
+      launch_pack_rows<S>(h, s, p, a, ntiles);
+    } else {
+      auto launch = [&](auto waves) {
+        constexpr int W = decltype(waves)::value, TPB = kStepWaves / W;
+        const int groups = (ntiles + TPB - 1) / TPB;
+        hipLaunchKernelGGL((k_step_pack<S, EAM, MATRIX, W>),
+                           dim3(step_pack_grid<EAM>(groups, h.num_cus)), dim3(kStepWaves * kWave),
+                           0, s, p, a, groups);
+      };
+      // Sixteen waves per tile while the tiles fill two blocks per CU, eight past that: us by
+      // waves per tile 2, 4, 8, 16 (float32, packed edges; four were used at every size before)
+      //   16 tiles (1,008 atoms)  49, 33, 22, 17*   1,024 tiles (65,536)   68, 49, 41*, 45
+      //   465 tiles (29,716)      58, 38, 28, 26*   2,048 tiles (131,072)  85, 75, 73*, 79
+      if (ntiles <= 2 * (h.num_cus > 0 ? h.num_cus : 256))
+        launch(std::integral_constant<int, 16>{});
+      else
+        launch(std::integral_constant<int, 8>{});
+    }
   }
   ++h.pack_serial;
   FusedPack fp;
@@ -659,7 +670,6 @@ static hipError_t pack_fused(Handle &h, hipStream_t s, const double *x, const in
   p.ghost_off = nullptr;  // no model: nothing to forward
   p.ghost_list = nullptr;
   const int ntiles = (num_rows + kWave - 1) / kWave;
-  const int ngroups = ntiles > 0 ? (ntiles + kStepTPB - 1) / kStepTPB : 1;
   // float64: the pack kernel writes the atom records itself, and the previous fused step's last
   // block left the pack state as the record launch would (h.pack_ready), else one block resets
   // it. float32 filters from the records (pack_keeps_f32), so they come first.
@@ -676,9 +686,7 @@ static hipError_t pack_fused(Handle &h, hipStream_t s, const double *x, const in
   }
   if (ntiles > 0) {
     StageTimer timer(h, s, "step_pack");
-    const int grid = step_pack_grid<false>(ngroups, h.num_cus);
-    hipLaunchKernelGGL((k_step_pack<S, false, false>), dim3(grid),
-                       dim3(kStepW * kStepTPB * kWave), 0, s, p, a, ngroups);
+    launch_pack_rows<S>(h, s, p, a, ntiles);
   }
   ++h.pack_serial;
   out->state = h.d_pack_state;
