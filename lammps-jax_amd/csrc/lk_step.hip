@@ -480,11 +480,217 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
   }
 }
 
-// The pack alone (two-sided and LJ steps).
+// The pack alone (two-sided and LJ steps; no model in the loop) of rows of up to 256 slots: one
+// 64-row tile per block of eight waves, wave w walking the slots w, w + 8, ... of every row. What
+// bounds it is the round trips of the walk (a list entry, then its neighbour's position), so four
+// slots go at a time: their records gather together while the next four entries load, and every
+// load is unconditional, so waiting for one never waits for a later one. The walked neighbours
+// stay in LDS for the compacted write: read from memory again, each batch's loads wait for the
+// stores of the batch before (one counter retires both in order). Blocks of one tile instead of
+// four overlap one tile's walk with another's write, and small lists reach more CUs; eight waves
+// against four halve the rounds of a tile. us before (k_step_pack's 4 tiles of 4 waves) and after:
+//   1,024 atoms LJ float64 21 -> 9.8            1,048,576 atoms half list float32 292 -> 238
+//   8,192 atoms half list float64 24 -> 10.7    262,144 atoms LJ with ghost rows float32 169 -> 131
+//   131,072 atoms half list float64 53 -> 35    (about 2.5 TB/s of list and packed edges)
+// Measured beside it: two slots at a time 254 and 140 (the last two float32 cases), four waves 226
+// and 147, sixteen 319 and 153, the edges compacted in LDS and stored 16 bytes at a time 238 and
+// 131.
+constexpr int kPackW = 8;      // waves per tile
+constexpr int kPackU = 4;      // slots of a row in flight per wave
+constexpr int kPackKeep = 128; // slots whose neighbours stay in LDS: 32 KB, four blocks per CU
+
+template <typename S>
+__global__ __launch_bounds__(kPackW * kWave) __attribute__((amdgpu_waves_per_eu(8))) LK_EIGHT_WAVES
+void k_pack_rows(StepPack p, const Atom4<S> *__restrict__ atoms, int nlocal,
+                 double *__restrict__ partials, int ntiles)
+{
+  constexpr int W = kPackW, U = kPackU, KEEP = kPackKeep;
+  static_assert(32 % (W * U) == 0, "a round's slots lie in one validity word");
+  __shared__ int sent[KEEP][kWave];  // the neighbours of the walked slots
+  __shared__ uint32_t sbits[kStepMaxWords][kWave];
+  __shared__ int sbase;
+  if constexpr (sizeof(S) == 8) {
+    // the atom records for the sweeps (cpp:35-52: x as is, species = type - 1)
+    if (p.atoms_out)
+      for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < p.records;
+           i += gridDim.x * blockDim.x) {
+        const int sp = p.type[i] - 1;
+        Atom4<double> r;
+        r.x = p.x[3L * i + 0];
+        r.y = p.x[3L * i + 1];
+        r.z = p.x[3L * i + 2];
+        r.w = static_cast<double>(sp);
+        p.atoms_out[i] = r;
+        p.species_out[i] = sp;
+      }
+  }
+  const int tile = tile_of_block();
+  if (tile >= ntiles) return;  // whole block
+  const int wave = wave_in_block();
+  const int lane = threadIdx.x & (kWave - 1);
+  const int ii = tile * kWave + lane;
+  const bool row = ii < p.num_rows;
+  int i = -1, nn = 0;
+  if (row) {
+    i = p.ilist[ii];
+    if (i < p.max_atoms)
+      nn = min(p.numneigh[i], p.maxneighs);
+    else
+      i = -1;  // cpp:84: rows past max_atoms pack nothing
+  }
+  const int nn_max = wave_max_int(nn);
+  const int nwords = (nn_max + 31) >> 5;  // at most kStepMaxWords (launch_pack_rows)
+  for (int w = wave; w < nwords; w += W) sbits[w][lane] = 0u;
+  double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
+  Atom4<float> xa{0.0f, 0.0f, 0.0f, 0.0f};
+  if (i >= 0) {
+    xi0 = p.x[3L * i + 0];
+    xi1 = p.x[3L * i + 1];
+    xi2 = p.x[3L * i + 2];
+    if constexpr (sizeof(S) == 4) xa = atoms[i];
+  }
+  const float sa = fabsf(xa.x) + fabsf(xa.y) + fabsf(xa.z);
+  __syncthreads();
+  if (wave < nn_max) {
+    // The row of a lane whose slots reach nn_max: every slot below it exists there, so a lane
+    // past its own row reads that one (unused) and the loads need no branch.
+    const int longest = __shfl(i, __builtin_ctzll(wave_ballot(nn == nn_max)), kWave);
+    auto slot_entry = [&](int jj) -> int {
+      const int at = min(jj, nn_max - 1);  // uniform
+      const int *col = p.neighbors + static_cast<long>(at) * p.stride;
+      return col[static_cast<unsigned>(at < nn ? i : longest)] & kNeighMask;
+    };
+    struct Near {
+      double x0, x1, x2;
+    };
+    using Rec = std::conditional_t<sizeof(S) == 4, Atom4<float>, Near>;
+    auto gather = [&](int jj, int j) -> Rec {
+      const long q = (jj < nn && j < p.max_atoms) ? j : 0;
+      if constexpr (sizeof(S) == 4) {
+        return atoms[q];
+      } else {
+        Near r;
+        r.x0 = p.x[3 * q + 0];
+        r.x1 = p.x[3 * q + 1];
+        r.x2 = p.x[3 * q + 2];
+        return r;
+      }
+    };
+    int e[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) e[q] = slot_entry(wave + q * W);
+    for (int jj = wave; jj < nn_max; jj += U * W) {
+      Rec r[U];
+      int ne[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) r[q] = gather(jj + q * W, e[q]);
+#pragma unroll
+      for (int q = 0; q < U; ++q) ne[q] = slot_entry(jj + (U + q) * W);
+      uint32_t part = 0;
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int slot = jj + q * W, j = e[q];
+        bool keep = slot < nn && j < p.max_atoms;
+        if constexpr (sizeof(S) == 4) {
+          if (keep) keep = pack_keeps_f32(p, xa, sa, r[q], j, xi0, xi1, xi2);
+        } else {
+#pragma clang fp contract(off)
+          const double dx = xi0 - r[q].x0, dy = xi1 - r[q].x1, dz = xi2 - r[q].x2;
+          // PackNeighborFunctor keeps rsq <= cutsq (cpp:84-101)
+          keep = keep && !(dx * dx + dy * dy + dz * dz > p.cutsq);
+        }
+        part |= keep ? 1u << (slot & 31) : 0u;
+        if (slot < KEEP) sent[slot][lane] = j;
+        e[q] = ne[q];
+      }
+      if (part) atomicOr(&sbits[jj >> 5][lane], part);
+    }
+  }
+  __syncthreads();
+  int c = 0;
+  for (int w = 0; w < nwords; ++w) c += __popc(sbits[w][lane]);
+  const int total = wave_sum(c);
+  if (wave == 0) {
+    if (row) {
+      p.row_count[ii] = c;
+      p.row_atom[ii] = i;
+    }
+    const uint64_t gmask = wave_ballot(i >= nlocal && c > 0);
+    if (lane == 0) {
+      // the tile's slots [base, base + total): one claim per tile (cpp:102-110 claims per entry)
+      const int base = atomicAdd(&p.state[kDemand], total);
+      sbase = base;
+      p.tile_base[tile] = base;
+      if (gmask != 0) atomicOr(&p.state[kGhostFlag], 1);
+      put_partial(partials + 8L * tile + 0, 0.0);
+    }
+  }
+  if (row)
+    for (int w = wave; w < nwords; w += W)
+      p.bits[static_cast<long>(w) * p.pitch + ii] = sbits[w][lane];
+  // Compacted write, as k_step_pack's: wave w writes one contiguous range of ordinals.
+  const int kmax = wave_max_int(c);
+  const int per = (kmax + W - 1) / W;
+  const int k0 = min(wave * per, kmax);
+  const int k1 = min(k0 + per, kmax);
+  int cursor = wave_sum(min(c, k0));
+  int wd = 0;
+  uint32_t word = 0;
+  if (k0 < c) {
+    word = sbits[0][lane];
+    int skip = k0;
+    while (skip > 0) {
+      const int pc = __popc(word);
+      if (pc <= skip) {  // the k0-th entry lies in a later word
+        skip -= pc;
+        word = sbits[++wd][lane];
+      } else {
+        for (; skip > 0; --skip) word &= word - 1u;
+      }
+    }
+  }
+  __syncthreads();
+  const int base = sbase;
+  constexpr int B = 4;
+  for (int k = k0; k < k1; k += B) {
+    int jv[B], ev[B];
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const bool active = k + q < k1 && k + q < c;
+      const uint64_t M = wave_ballot(active);
+      const int at = base + cursor + lanes_below(M);
+      cursor += __popcll(M);
+      ev[q] = active && at < p.max_edges ? at : -1;  // past the capacity the count is the demand
+      jv[q] = 0;
+      if (active) {
+        while (word == 0) word = sbits[++wd][lane];
+        const int jj = wd * 32 + __builtin_ctz(word);
+        word &= word - 1u;
+        jv[q] = jj < KEEP ? sent[jj][lane]
+                          : p.neighbors[static_cast<long>(jj) * p.stride + i] & kNeighMask;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      if (ev[q] >= 0) {
+        p.receivers[ev[q]] = jv[q];
+        p.senders[ev[q]] = i;
+        p.mask[ev[q]] = 1;
+      }
+    }
+  }
+}
+
+// Rows of more than 256 slots, whose validity words LDS does not hold, take k_step_pack.
 template <typename S>
 static void launch_pack_rows(Handle &h, hipStream_t s, const StepPack &p, const EamArgs<S> &a,
                              int ntiles)
 {
+  if (p.maxneighs <= 32 * kStepMaxWords) {
+    hipLaunchKernelGGL((k_pack_rows<S>), dim3(tile_grid(ntiles)), dim3(kPackW * kWave), 0, s, p,
+                       a.atoms, a.nlocal, a.partials, ntiles);
+    return;
+  }
   constexpr int W = 8, TPB = kStepWaves / W;
   const int ngroups = (ntiles + TPB - 1) / TPB;
   hipLaunchKernelGGL((k_step_pack<S, false, false, W>),
