@@ -2,7 +2,8 @@
 
 `k_pack_rows` (two-sided and LJ steps) keeps the neighbours of 128 slots of a row in LDS and reads
 later ones again, four slots of eight waves at a time; lists with room for more than 256 slots take
-`k_step_pack`, whose bits past 256 slots stay in memory. The rows are cut to, or given far atoms up
+`k_step_pack`, whose bits past 256 slots stay in memory. `k_pack_count` and `k_pack_write` (the pack
+called on its own) go 256 slots at a time. The rows are cut to, or given far atoms up
 to, the lengths under test (the far ones are dropped by the cutoff, so the packed pairs come from
 either side of each edge), and the last tile is partly filled. The float32 one-sided EAM step's pack
 decides from float records, so a whole neighbour shell is put on its cutoff. Packed pairs bit for
@@ -78,8 +79,8 @@ def test_pack_rows(gpu, scheme, precision, cells, longest, width):
                        mask=m, precision=precision,
                        mode=O.PLAIN if scheme == "plain" else O.ONESIDED)
     rows = sysm.nall if scheme == "plain" else sysm.nlocal
-    for _ in range(2):
-        info = pj.compute()
+    for fused in (True, False, True):  # False: the three entry points (k_pack_count, k_pack_write)
+        info = pj.compute(fused=fused)
         assert info.edge_count == count and info.edge_overflow == 0
         np.testing.assert_array_equal(canonical(*pj.edges()), canonical(s, r, m))
         assert_energy(precision, info.energy, ref["energy"], sysm.nlocal)
