@@ -39,7 +39,7 @@ namespace lk {
 
 constexpr int kTileSortN = 2048;      // bitonic sort width of the union build (>= kTileUnion)
 constexpr int kTileHash = 8192;       // hash slots of the union build
-constexpr int kTileW = 6;             // waves per sub-tile
+constexpr int kTileW = 6;             // waves per sub-tile (twice that for a sub-tile alone)
 constexpr int kTileSub = kTileRows / kWave;
 constexpr int kTileBlocksPerCu = 2;   // 79.5 KB of LDS per block
 constexpr int kTileIdGroups = 40;     // slot groups per row whose ids the walk keeps in LDS
@@ -553,10 +553,14 @@ struct TileStep {
   int records;
 };
 
-__global__ __launch_bounds__(kTileW * kTileSub * kWave) __attribute__((amdgpu_waves_per_eu(6)))
+// SUB: the 64-row sub-tiles of a tile that a block takes (both, or one: two blocks per tile, each
+// staging the whole union); W waves per sub-tile.
+template <int W, int SUB>
+__global__ __launch_bounds__(W * SUB * kWave) __attribute__((amdgpu_waves_per_eu(6)))
 void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
 {
-  constexpr int W = kTileW, SUB = kTileSub;
+  constexpr int kParts = kTileSub / SUB;  // blocks per tile
+  constexpr int kRows = SUB * kWave;
   __shared__ double ux[kTileUnion], uy[kTileUnion], uz[kTileUnion];
   __shared__ uint32_t ugid[kTileUnion];  // atom id | species << 24
   __shared__ uint32_t sbits[SUB][kTileMaxSlots / 32][kWave];
@@ -564,11 +568,11 @@ void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
   __shared__ int sbase[SUB];
   // the ids of the walked slot groups, for the compacted write (groups past kTileIdGroups are
   // read again from the tile list)
-  __shared__ uint64_t sids[kTileIdGroups][kTileRows];
-  // the walk's partial counts and densities reuse ux once every wave has left the walk
+  __shared__ uint64_t sids[kTileIdGroups][kRows];
+  // the walk's partial counts and densities reuse ux and uy once every wave has left the walk
   int(*cpart)[W][kWave] = reinterpret_cast<int(*)[W][kWave]>(ux);
-  double(*rpart)[W][kWave] = reinterpret_cast<double(*)[W][kWave]>(ux + SUB * W * kWave / 2);
-  static_assert(SUB * W * kWave * 3 <= 2 * kTileUnion, "the partials fit in ux");
+  double(*rpart)[W][kWave] = reinterpret_cast<double(*)[W][kWave]>(uy);
+  static_assert(SUB * W * kWave <= kTileUnion, "the partials fit in ux and uy");
   constexpr int kBitWords = SUB * (kTileMaxSlots / 32) * kWave;
 
   // the density intervals are read from the density-only (f, d) table in memory (no LDS window)
@@ -589,12 +593,13 @@ void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
       p.atoms_out[i] = r;
       p.species_out[i] = sp;
     }
-  for (GroupWalk gw = group_walk(t.ntiles); gw.g < gw.g_end; gw.g += gw.step) {
-    const int tile = gw.g;
+  for (GroupWalk gw = group_walk(t.ntiles * kParts); gw.g < gw.g_end; gw.g += gw.step) {
+    const int tile = gw.g / kParts;
+    const int tsub = gw.g % kParts * SUB + sub;  // this wave's sub-tile in the tile
     const int U = t.ucount[tile];
     const bool staged = U >= 0;  // block-uniform
     // the tile's rows, loaded first so that their round trips overlap the union's staging
-    const int pos = tile * kTileRows + sub * kWave + lane;
+    const int pos = tile * kTileRows + tsub * kWave + lane;
     const int i = t.atom[pos];
     const int nn = t.nn[pos];
     double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
@@ -629,7 +634,7 @@ void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
       // bits of its groups in one bit word and ORs it into LDS when it moves to another word.
       const int ngroups = (nmax + 3) >> 2;
       const uint64_t *lidp =
-          t.lid + static_cast<long>(tile) * t.groups * kTileRows + sub * kWave + lane;
+          t.lid + static_cast<long>(tile) * t.groups * kTileRows + tsub * kWave + lane;
       uint64_t ids = wave < ngroups ? lidp[static_cast<long>(wave) * kTileRows] : 0;
       uint32_t word = 0;
       int wd = wave >> 3;
@@ -699,7 +704,7 @@ void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
     cpart[sub][wave][lane] = cnt;
     rpart[sub][wave][lane] = rho;
     __syncthreads();
-    const int subtile = tile * SUB + sub;
+    const int subtile = tile * kTileSub + tsub;
     if (wave == 0) {
       cnt = cpart[sub][0][lane];
       rho = rpart[sub][0][lane];
@@ -790,7 +795,7 @@ void k_step_tiles(TileStep p, EamArgs<double> a, TileView t)
                   (jj >> 2) < kTileIdGroups
                       ? sids[jj >> 2][sub * kWave + lane]
                       : t.lid[((static_cast<long>(tile) * t.groups + (jj >> 2)) * kTileRows) +
-                              sub * kWave + lane];
+                              tsub * kWave + lane];
               j = static_cast<int>(ugid[static_cast<uint32_t>(w4 >> (16 * (jj & 3))) & 0xFFFFu] &
                                    0xFFFFFFu);
             } else {
@@ -1003,8 +1008,22 @@ hipError_t launch_step_tiles(Handle &h, hipStream_t s, const double *x, const in
   t.ntiles = (num_rows + kTileRows - 1) / kTileRows;
   (void)nlocal;
   StageTimer timer(h, s, "step_pack");
-  const int grid = persistent_grid(t.ntiles, kTileBlocksPerCu, h.num_cus);
-  hipLaunchKernelGGL(k_step_tiles, dim3(grid), dim3(kTileW * kTileSub * kWave), 0, s, p, a, t);
+  auto launch = [&](auto waves, auto subs) {
+    constexpr int W = decltype(waves)::value, SUB = decltype(subs)::value;
+    const int grid = persistent_grid(t.ntiles * (kTileSub / SUB), kTileBlocksPerCu, h.num_cus);
+    hipLaunchKernelGGL((k_step_tiles<W, SUB>), dim3(grid), dim3(W * SUB * kWave), 0, s, p, a, t);
+  };
+  // Up to one tile per CU, each 64-row half of a tile takes a block of its own: both blocks stage
+  // the tile's union, but twice the waves walk and write its rows and every CU still holds them all
+  // at once. us, whole tiles and halves (chosen starred):
+  //   8 tiles (1,008 atoms) 21.1, 15.3*   128 (16,384) 23.0, 17.4*   233 (29,716) 26.9, 23.2*
+  //   352 (45,056) 57.5*, 52.4            512 (65,536) 38.3*, 42.0   1,024 (131,072) 68.1*, 79.9
+  // (Halves of eight waves: 16.4, 18.7, 23.7 at the first three; of sixteen, one block per CU: 15.4,
+  // 17.8, 31.2.)
+  if (t.ntiles <= (h.num_cus > 0 ? h.num_cus : 256))
+    launch(std::integral_constant<int, 2 * kTileW>{}, std::integral_constant<int, 1>{});
+  else
+    launch(std::integral_constant<int, kTileW>{}, std::integral_constant<int, kTileSub>{});
   return hipGetLastError();
 }
 
