@@ -6,9 +6,9 @@
 // virial (eam.py:385-398, cpp:175-245).
 //
 //   K0 atoms:  atom records and species (lk_pack.hip); clears the pack's demand counter.
-//   K1 pack:   per 64-row tile, the list walk with the cutoff filter (float64: positions
-//              gathered from the records, one 32-byte load per entry), validity bits and row
-//              counts; on kept pairs the density of the row (float64: from the same r^2 the
+//   K1 pack:   per 64-row tile, the list walk with the cutoff filter (positions gathered from the
+//              records, one load of 32 bytes, or of 16 in float32, per entry), validity bits and
+//              row counts; on kept pairs the density of the row (float64: from the same r^2 the
 //              filter formed); then F(rho), F'(rho), F' copied to the row's ghost images (the
 //              forward comm of one rank) and the embedding energy of the tile. The tile then
 //              claims its slot range with one atomic add on the demand counter (the reference's

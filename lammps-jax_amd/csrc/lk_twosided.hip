@@ -294,7 +294,7 @@ constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 // of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
 constexpr int kBinLog = 6;
 constexpr int kBinAtoms = 1 << kBinLog;  // at most
-constexpr int kBinTiles = 8, kBinW = 2;  // a block's 64-row tiles and the waves of each
+constexpr int kBinWaves = 16;            // waves of a counting block: kBinWaves / W 64-row tiles
 constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
 constexpr int kBinProbes = 8;
 
@@ -328,19 +328,19 @@ __global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
 }
 
 // Count (SCATTER false: the in- and out-entries of each bin; also out_n and row_of) and scatter.
-// One lane per row, the waves of a tile sharing its slots; entries of adjacent lanes in the same
+// One lane per row, the W waves of a tile sharing its slots; entries of adjacent lanes in the same
 // bin (adjacent rows' k-th neighbours mostly are) count as one run, so a wave does one LDS update
 // per run.
-template <bool SCATTER, typename E>
-__global__ __launch_bounds__(kBinTiles *kBinW *kWave) LK_EIGHT_WAVES
+template <bool SCATTER, typename E, int W>
+__global__ __launch_bounds__(kBinWaves *kWave) LK_EIGHT_WAVES
 void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
 {
   __shared__ int tag[kBinTable], cnt[kBinTable];
   __shared__ int aux[kBinTable];  // count: out-entries; scatter: the block's first place
-  constexpr int kThreads = kBinTiles * kBinW * kWave;
+  constexpr int kThreads = kBinWaves * kWave, kTiles = kBinWaves / W;
   const int wave = wave_in_block(), lane = threadIdx.x & (kWave - 1);
-  const int wq = wave % kBinW;
-  const int ii = (blockIdx.x * kBinTiles + wave / kBinW) * kWave + lane;
+  const int wq = wave % W;
+  const int ii = (blockIdx.x * kTiles + wave / W) * kWave + lane;
   for (int k = threadIdx.x; k < kBinTable; k += kThreads) {
     tag[k] = -1;
     cnt[k] = 0;
@@ -370,19 +370,19 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   }
   auto walk = [&](auto &&use) {
     constexpr int kBatch = 8;
-    for (int j0 = wq; j0 < nmax; j0 += kBinW * kBatch) {
+    for (int j0 = wq; j0 < nmax; j0 += W * kBatch) {
       int raw[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        const int jj = j0 + kBinW * u;
+        const int jj = j0 + W * u;
         raw[u] = jj < nn ? L.neighbors[static_cast<long>(jj) * L.stride + i] : 0;
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        if (j0 + kBinW * u >= nmax) break;  // wave-uniform
+        if (j0 + W * u >= nmax) break;  // wave-uniform
         const int j = raw[u] & kNeighMask;
         // list_neighbor's filter on the loaded entry
-        const bool ok = j0 + kBinW * u < nn && j < L.max_atoms && !(L.half_filter && j < i);
+        const bool ok = j0 + W * u < nn && j < L.max_atoms && !(L.half_filter && j < i);
         const int b = ok ? j >> L.bin_log : -1;
         const int before = __shfl_up(b, 1, kWave);
         const bool head = lane == 0 || before != b;
@@ -1480,21 +1480,43 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   B.out = B.next + B.n;
   B.off = B.out + B.n;
   B.loff = B.off + B.n + 1;
-  const dim3 row_grid((L.rows + kBinTiles * kWave - 1) / (kBinTiles * kWave));
-  constexpr int kRowThreads = kBinTiles * kBinW * kWave;
+  // Waves per 64-row tile of the counting blocks: many where the tiles are few, so that the blocks
+  // reach the CUs; two past eight tiles per CU, where a block's eight tiles share the bins they
+  // name and so its LDS counts (fewer claims in memory). Count and scatter together in us by waves
+  // 2, 4, 8, 16, chosen starred; two at every size before:
+  //   16 tiles (1,024 rows, plain)  65, 38, 26, 20*    1,024 tiles (65,536, plain) 81, 57*, 62, 88
+  //   128 tiles (8,192, half)       61, 37, 27*, 25    2,048 tiles (131,072, half) 74, 56*, 75, 98
+  //   500 tiles (32,000, plain)     76, 51, 45*, 53    4,000 tiles (256,000, half) 105*, 117, 134, 163
+  const int cus = h.num_cus > 0 ? h.num_cus : 256, tiles = (L.rows + kWave - 1) / kWave;
+  auto bins = [&](auto scatter, auto *tmp) {
+    using E = std::remove_pointer_t<decltype(tmp)>;
+    auto launch = [&](auto waves) {
+      constexpr int W = decltype(waves)::value, kTiles = kBinWaves / W;
+      hipLaunchKernelGGL((k_inc_bins<decltype(scatter)::value, E, W>),
+                         dim3((tiles + kTiles - 1) / kTiles), dim3(kBinWaves * kWave), 0, s, L, B,
+                         tmp);
+    };
+    if (4 * tiles <= cus)
+      launch(std::integral_constant<int, 16>{});
+    else if (tiles <= 2 * cus)
+      launch(std::integral_constant<int, 8>{});
+    else if (tiles <= 8 * cus)
+      launch(std::integral_constant<int, 4>{});
+    else
+      launch(std::integral_constant<int, 2>{});
+  };
   {
     StageTimer timer(h, s, "inc_count");
     hipLaunchKernelGGL(k_inc_clear, dim3((atoms + 255) / 256), dim3(256), 0, s, L, B);
     if (L.rows > 0)
-      hipLaunchKernelGGL((k_inc_bins<false, uint32_t>), row_grid, dim3(kRowThreads), 0, s, L, B,
-                         static_cast<uint32_t *>(nullptr));
+      bins(std::false_type{}, static_cast<uint32_t *>(nullptr));
     hipLaunchKernelGGL(k_inc_bin_scan, dim3(1), dim3(kScanThreads), 0, s, B);
   }
   auto finish = [&](auto *tmp) {
     using E = std::remove_pointer_t<decltype(tmp)>;
     if (L.rows > 0) {
       StageTimer timer(h, s, "inc_fill");
-      hipLaunchKernelGGL((k_inc_bins<true, E>), row_grid, dim3(kRowThreads), 0, s, L, B, tmp);
+      bins(std::true_type{}, tmp);
     }
     StageTimer timer(h, s, "inc_place");
     if (fold)
