@@ -148,7 +148,8 @@ int ensure_incidence(Handle &h, long entries = 0)
     h.d_inc_tmp = nullptr;
     h.d_inc = nullptr;
     h.inc_cap = 0;
-    if ((e = dalloc(&h.d_inc_tmp, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence staging)");
+    const long words = h.contract.max_atoms <= lk::kBinAtoms32 ? need : need + (need + 1) / 2;
+    if ((e = dalloc(&h.d_inc_tmp, words)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence staging)");
     if ((e = dalloc(&h.d_inc, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lists)");
     h.inc_cap = need;
     h.inc_key = Handle::IncKey{};  // rebuild

@@ -47,6 +47,10 @@ struct FusedPack {
   int pad = 0;           // padding index (max_atoms)
 };
 
+// List-built incidence entries on their way hold atom and place in 32 bits up to this many atoms,
+// in 64 past it.
+constexpr long kBinAtoms32 = (1L << 26) - 1;
+
 struct Handle {
   lk_contract contract{};
   int accum = LK_ACCUM_PLAIN;
@@ -134,7 +138,8 @@ struct Handle {
                                 // each atom's row for the list-built ones
   int *d_inc_loc = nullptr;     // [max_atoms + 1] offsets within each scan chunk
   int *d_inc_part = nullptr;    // [chunks] chunk offsets
-  uint32_t *d_inc_tmp = nullptr;  // [inc_cap] entries on their way into d_inc
+  uint32_t *d_inc_tmp = nullptr;  // entries on their way into d_inc: [inc_cap] words, half as many
+                                  // again past kBinAtoms32 atoms
   int *d_inc = nullptr;         // [inc_cap] other atom | side << 31: all of an edge-built list's
                                 // entries in edge order, a list-built one's in-entries
   int *d_inc_len = nullptr;     // [max_atoms + 1] entries of each atom in d_inc
