@@ -236,6 +236,13 @@ __global__ __launch_bounds__(256) void k_inc_sort(IncArgs a, int nsort)
 // j >= max_atoms, the half filter j < i); its distance filter is applied each step. Atom a's
 // list is its out-entries (the kept slots of its own row, in slot order: other = j) followed by
 // its in-entries (slots of other rows naming a: other = i, side bit set) in ascending i.
+
+// How the bins of the build are laid out (k_inc_lists).
+struct BinLayout {
+  int bin_log;   // atoms per bin: 1 << bin_log
+  int per_atom;  // in-entries kept in LDS per atom; 0: none, the bins sort theirs
+  int pitch;     // slots per staged row
+};
 struct ListArgs {
   const int *ilist;
   const int *numneigh;
@@ -252,7 +259,10 @@ struct ListArgs {
   int *len;     // entries of each atom
   int *inc;
   uint32_t *claim;  // the sorted path's marks where LDS does not hold them, a word per in-entry
-  int bin_log;      // atoms per bin: 1 << bin_log
+  int fold;         // the plain scheme's fold
+  BinLayout layout;
+  int *longest;  // lists with room for longer rows than 64-atom bins take: the longest row, which
+                 // the layout then goes by; else null
 };
 
 // The row atom of list row ii and its slot count, or -1 when the row packs nothing.
@@ -295,6 +305,8 @@ constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 // of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
 constexpr int kBinLog = 6;
 constexpr int kBinAtoms = 1 << kBinLog;  // at most
+constexpr int kBinLeastLog = 2;
+constexpr int kBinPool = 62 * 1024;      // LDS of a bin's lists (two blocks or more share a CU)
 constexpr int kBinWaves = 16;            // waves of a counting block: kBinWaves / W 64-row tiles
 constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
 constexpr int kBinProbes = 8;
@@ -304,9 +316,48 @@ constexpr int kBinProbes = 8;
 template <typename E>
 constexpr int kBinShift = sizeof(E) == 4 ? 26 : 32;
 
-// The bins' counters and offsets, [bins] each (offsets [bins + 1]).
+// Atoms per bin: 64, or fewer where the out-entries of that many rows and their in-entries (with
+// a fold, hash tables four fifths full at the longest row's length) would take more than kBinPool.
+// Rows past 1,763 slots (1,981 without a fold) keep bins of four atoms and sort.
+__host__ __device__ inline BinLayout bin_layout(long longest, bool fold)
+{
+  const long per = fold ? (longest * 5 / 4 + 7) / 4 * 4 : (longest + 7) / 4 * 4;
+  const long pitch = longest | 1;
+  BinLayout y{kBinLog, 0, 0};
+  while (y.bin_log > kBinLeastLog && (4 * (per + pitch)) << y.bin_log > kBinPool) --y.bin_log;
+  if ((4 * (per + pitch)) << y.bin_log <= kBinPool) {
+    y.per_atom = static_cast<int>(per);
+    y.pitch = static_cast<int>(pitch);
+  }
+  return y;
+}
+
+// An engine's list may have room for far more slots than its rows have, so where the room alone
+// would make the bins smaller the rows are measured on the device first. By the room, the step on a
+// new list of 32,000 LJ atoms with 80 slots a row (plain) took 245 us at room for 240 slots, 998 at
+// 700 and 6,390 at 1,700; by the rows it takes 164 at each (153 at room for 80).
+__device__ __forceinline__ BinLayout bin_layout_of(const ListArgs &L)
+{
+  return L.longest ? bin_layout(*L.longest, L.fold != 0) : L.layout;
+}
+
+__device__ __forceinline__ int bin_count(const ListArgs &L, const BinLayout &y)
+{
+  return (L.max_atoms + (1 << y.bin_log) - 1) >> y.bin_log;
+}
+
+__global__ __launch_bounds__(256) void k_inc_longest(ListArgs L)
+{
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x;
+  int nn = 0;
+  if (ii < L.rows) list_row(L, ii, nn);
+  const int most = wave_max_int(nn);
+  if ((threadIdx.x & (kWave - 1)) == 0 && most > 0) atomicMax(L.longest, most);
+}
+
+// The bins' counters and offsets, [cap] each (offsets [cap + 1]).
 struct Bins {
-  int n;
+  int cap;    // bins there is room for
   int *next;  // in-entries, then the scatter's next free place
   int *out;   // out-entries (list slots)
   int *off;   // first in-entry in the scatter's output
@@ -320,7 +371,7 @@ __global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
     L.out_n[i] = 0;
     L.row_of[i] = -1;
   }
-  if (i < B.n) {
+  if (i < B.cap) {
     B.next[i] = 0;
     B.out[i] = 0;
   }
@@ -349,6 +400,7 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   int nn = 0, i = -1;
   if (ii < L.rows) i = list_row(L, ii, nn);
   const int nmax = wave_max_int(nn);
+  const int bin_log = bin_layout_of(L).bin_log;
   __syncthreads();
   // the LDS slot of bin b, or -1 when the probed slots hold other bins (they keep them: the same
   // answer in both walks of the scatter)
@@ -365,8 +417,8 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   if (!SCATTER && wq == 0 && i >= 0) {
     L.out_n[i] = nn;
     L.row_of[i] = ii;
-    const int q = slot_of(i >> L.bin_log);
-    atomicAdd(q >= 0 ? &aux[q] : &B.out[i >> L.bin_log], nn);
+    const int q = slot_of(i >> bin_log);
+    atomicAdd(q >= 0 ? &aux[q] : &B.out[i >> bin_log], nn);
   }
   auto walk = [&](auto &&use) {
     constexpr int kBatch = 8;
@@ -383,7 +435,7 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
         const int j = raw[u] & kNeighMask;
         // list_neighbor's filter on the loaded entry
         const bool ok = j0 + W * u < nn && j < L.max_atoms && !(L.half_filter && j < i);
-        const int b = ok ? j >> L.bin_log : -1;
+        const int b = ok ? j >> bin_log : -1;
         const int before = __shfl_up(b, 1, kWave);
         const bool head = lane == 0 || before != b;
         const uint64_t heads = wave_ballot(head);
@@ -424,25 +476,26 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
       }
       at = __shfl(at, first, kWave) + lane - first;
       if (b >= 0)
-        tmp[at] = (static_cast<E>(j & ((1 << L.bin_log) - 1)) << kBinShift<E>) | static_cast<E>(i);
+        tmp[at] = (static_cast<E>(j & ((1 << bin_log) - 1)) << kBinShift<E>) | static_cast<E>(i);
     });
   }
 }
 
 // Exclusive scans of the bins' in-entries (off, and next in place) and of all their entries (loff),
 // one block.
-__global__ __launch_bounds__(kScanThreads) void k_inc_bin_scan(Bins B)
+__global__ __launch_bounds__(kScanThreads) void k_inc_bin_scan(ListArgs L, Bins B)
 {
+  const int nbins = bin_count(L, bin_layout_of(L));
   __shared__ int wsum[2][kScanThreads / kWave];
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
   int carry = 0, carry_l = 0;
-  for (int b0 = 0; b0 < B.n; b0 += kScanChunk) {
+  for (int b0 = 0; b0 < nbins; b0 += kScanChunk) {
     int v[kScanItems], w[kScanItems], s = 0, sl = 0;
 #pragma unroll
     for (int q = 0; q < kScanItems; ++q) {
       const int k = b0 + t * kScanItems + q;
-      v[q] = k < B.n ? B.next[k] : 0;
-      w[q] = k < B.n ? v[q] + B.out[k] : 0;
+      v[q] = k < nbins ? B.next[k] : 0;
+      w[q] = k < nbins ? v[q] + B.out[k] : 0;
       s += v[q];
       sl += w[q];
     }
@@ -470,7 +523,7 @@ __global__ __launch_bounds__(kScanThreads) void k_inc_bin_scan(Bins B)
 #pragma unroll
     for (int q = 0; q < kScanItems; ++q) {
       const int k = b0 + t * kScanItems + q;
-      if (k < B.n) {
+      if (k < nbins) {
         B.next[k] = run;
         B.off[k] = run;
         B.loff[k] = run_l;
@@ -480,7 +533,7 @@ __global__ __launch_bounds__(kScanThreads) void k_inc_bin_scan(Bins B)
     }
     __syncthreads();
   }
-  if (t == 0) B.off[B.n] = carry;
+  if (t == 0) B.off[nbins] = carry;
 }
 
 __device__ __forceinline__ uint32_t bin_hash(uint32_t atom, uint32_t slots)
@@ -533,7 +586,7 @@ __device__ __forceinline__ void store_ranked(const uint32_t *slots, int n, int c
 // out-entries look up their reverse (one that finds it is marked, and the in-entry leaves). The
 // out-entries are written without their gaps, what is left of the in-entries ranked by row atom.
 // A bin whose in-entries do not fit, one with a row that names an atom twice and whose reverse is
-// there, and every bin when per_atom is 0, sorts its in-entries instead (in LDS where they fit its
+// there, and every bin when `per_atom` is 0, sorts its in-entries instead (in LDS where they fit its
 // `pool_words`, else where they are) and finds them by bisection. By either path the m-th slot of a
 // row naming an atom pairs with the m-th slot of that atom's row naming it back.
 // A search of the bin's rows and entries for each entry stood in place of the sort: with rows of
@@ -588,7 +641,7 @@ __device__ __forceinline__ int lower_bound(const E *T, int n, E v)
 
 template <typename E, bool FOLD>
 __global__ __launch_bounds__(kListThreads) LK_EIGHT_WAVES
-void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int per_atom, int pitch, int pool_words)
+void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
 {
   extern __shared__ __align__(16) uint32_t pool[];  // [atoms][per_atom], then [atoms][pitch]
   __shared__ int nin[kBinAtoms], nout[kBinAtoms], rown[kBinAtoms];
@@ -596,7 +649,10 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int per_atom, int pitc
   __shared__ int spill;
   constexpr int kWaves = kListThreads / kWave;
   const int tid = threadIdx.x, wave = wave_in_block(), lane = tid & (kWave - 1);
-  const int na = 1 << L.bin_log, a0 = blockIdx.x << L.bin_log;
+  const BinLayout y = bin_layout_of(L);
+  if (static_cast<int>(blockIdx.x) >= bin_count(L, y)) return;  // whole block
+  const int per_atom = y.per_atom, pitch = y.pitch;
+  const int na = 1 << y.bin_log, a0 = blockIdx.x << y.bin_log;
   const int e0 = B.off[blockIdx.x], n = B.off[blockIdx.x + 1] - e0;
   const int slots = na * per_atom;
   uint32_t *outs = pool + slots;
@@ -637,7 +693,7 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int per_atom, int pitc
     __syncthreads();
   };
   // thread t stages the slots t / na, + threads / na, ... of atom t % na
-  const int d_own = tid & (na - 1), q0 = tid >> L.bin_log, qstep = kListThreads >> L.bin_log;
+  const int d_own = tid & (na - 1), q0 = tid >> y.bin_log, qstep = kListThreads >> y.bin_log;
   if (per_atom > 0) {
     if constexpr (FOLD) {
       for (int e = tid; e < n; e += kListThreads) {
@@ -1589,31 +1645,27 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   L.len = h.d_inc_len;
   L.inc = h.d_inc;
   const int atoms = L.max_atoms;
-  // Atoms per bin: 64, or fewer where the out-entries of that many rows and their in-entries (with
-  // a fold, hash tables four fifths full at the list's width) would take more than 62 KB of LDS
-  // (two blocks or more share a CU). Rows past 1,700 slots go through memory.
-  constexpr long kPool = 62 * 1024;
-  const long per = fold ? (L.maxneighs * 5L / 4 + 7) / 4 * 4 : (L.maxneighs + 7L) / 4 * 4;
-  const int pitch = L.maxneighs | 1;
-  L.bin_log = kBinLog;
-  while (L.bin_log > 2 && 4 * (per + pitch) << L.bin_log > kPool) --L.bin_log;
-  const bool staged = 4 * (per + pitch) << L.bin_log <= kPool;
-  const int per_atom = staged ? static_cast<int>(per) : 0;
-  const size_t lds = staged ? static_cast<size_t>(4 * (per + pitch)) << L.bin_log : kPool;
+  L.fold = fold ? 1 : 0;
+  L.layout = bin_layout(L.maxneighs, fold);
   Bins B;
-  B.n = (atoms + (1 << L.bin_log) - 1) >> L.bin_log;
-  if (4L * B.n + 2 > h.bins_cap) {  // rarely: rows that need smaller bins; a build may be running
+  B.cap = (atoms + (1 << L.layout.bin_log) - 1) >> L.layout.bin_log;
+  const long words = 4L * B.cap + 2;
+  if (words > h.bins_cap) {  // rarely: a list with more room; a build may be running
     if (hipError_t e = hipDeviceSynchronize(); e != hipSuccess) return e;
     if (h.d_bins) (void)hipFree(h.d_bins);
     h.d_bins = nullptr;
     h.bins_cap = 0;
-    if (hipError_t e = hipMalloc(&h.d_bins, (4L * B.n + 2) * sizeof(int)); e != hipSuccess) return e;
-    h.bins_cap = 4L * B.n + 2;
+    if (hipError_t e = hipMalloc(&h.d_bins, words * sizeof(int)); e != hipSuccess) return e;
+    h.bins_cap = words;
   }
   B.next = h.d_bins;
-  B.out = B.next + B.n;
-  B.off = B.out + B.n;
-  B.loff = B.off + B.n + 1;
+  B.out = B.next + B.cap;
+  B.off = B.out + B.cap;
+  B.loff = B.off + B.cap + 1;
+  const bool measure = L.layout.bin_log < kBinLog;
+  L.longest = measure ? B.loff + B.cap : nullptr;
+  const size_t lds = measure ? kBinPool
+                             : static_cast<size_t>(4 * (L.layout.per_atom + L.layout.pitch)) << kBinLog;
   // Waves per 64-row tile of the counting blocks: many where the tiles are few, so that the blocks
   // reach the CUs; two past eight tiles per CU, where a block's eight tiles share the bins they
   // name and so its LDS counts (fewer claims in memory). Count and scatter together in us by waves
@@ -1641,10 +1693,15 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   };
   {
     StageTimer timer(h, s, "inc_count");
+    if (measure) {
+      hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(256), 0, s, L.longest, 1L);
+      if (L.rows > 0)
+        hipLaunchKernelGGL(k_inc_longest, dim3((L.rows + 255) / 256), dim3(256), 0, s, L);
+    }
     hipLaunchKernelGGL(k_inc_clear, dim3((atoms + 255) / 256), dim3(256), 0, s, L, B);
     if (L.rows > 0)
       bins(std::false_type{}, static_cast<uint32_t *>(nullptr));
-    hipLaunchKernelGGL(k_inc_bin_scan, dim3(1), dim3(kScanThreads), 0, s, B);
+    hipLaunchKernelGGL(k_inc_bin_scan, dim3(1), dim3(kScanThreads), 0, s, L, B);
   }
   auto finish = [&](auto *tmp) {
     using E = std::remove_pointer_t<decltype(tmp)>;
@@ -1654,11 +1711,11 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
     }
     StageTimer timer(h, s, "inc_place");
     if (fold)
-      hipLaunchKernelGGL((k_inc_lists<E, true>), dim3(B.n), dim3(kListThreads), lds, s, L, B, tmp,
-                         per_atom, pitch, static_cast<int>(lds / 4));
+      hipLaunchKernelGGL((k_inc_lists<E, true>), dim3(B.cap), dim3(kListThreads), lds, s, L, B,
+                         tmp, static_cast<int>(lds / 4));
     else
-      hipLaunchKernelGGL((k_inc_lists<E, false>), dim3(B.n), dim3(kListThreads), lds, s, L, B, tmp,
-                         per_atom, pitch, static_cast<int>(lds / 4));
+      hipLaunchKernelGGL((k_inc_lists<E, false>), dim3(B.cap), dim3(kListThreads), lds, s, L, B,
+                         tmp, static_cast<int>(lds / 4));
   };
   // d_inc_tmp holds an entry and a word of marks per list slot (ensure_incidence)
   L.claim = h.d_inc_tmp + static_cast<long>(L.rows) * L.maxneighs * (atoms <= kBinAtoms32 ? 1 : 2);

@@ -1,0 +1,82 @@
+"""The list-built incidence lists go by the rows of a list, not by the room it has for them.
+
+An engine's list may have room for far more slots than any row uses (it grows by the widest row ever
+seen). Past the room that bins of 64 atoms take (107 slots with the plain scheme's fold, 119
+without), the build measures the longest row first and sizes its bins by it: 64, 32, 16, 8 and 4
+atoms are reached here by rows given distinct atoms past the cutoff, each with tight room and with
+room for 2,500 slots. Against the oracle, and the same forces bit for bit at either room."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+from lk_testutil import assert_energy, assert_forces
+from lammps_jax_amd import harness, systems
+from lammps_jax_amd.pair import PairJax
+
+pytestmark = pytest.mark.gpu
+
+
+def _filled(sysm, cutoff, longest):
+    """The list with every fifth row given atoms past the cutoff up to `longest` slots."""
+    lst = dict(sysm.list)
+    stride, rows = lst["stride"], lst["maxneighs"]
+    num = np.array(lst["numneigh"], copy=True)
+    nb = np.zeros((max(rows, longest), stride), np.int32)
+    nb[:rows] = np.asarray(lst["neighbors"]).reshape(rows, stride)
+    x = sysm.x[:sysm.nall]
+    for i in np.asarray(lst["ilist"])[:lst["inum"]:5]:
+        far = np.sum((x - x[i]) ** 2, axis=1) > (cutoff + 0.1) ** 2
+        far[nb[:num[i], i] & 0x3FFFFFFF] = False
+        add = np.flatnonzero(far)[:max(0, longest - int(num[i]))]
+        nb[num[i]:num[i] + len(add), i] = add
+        num[i] += len(add)
+    room = int(num[np.asarray(lst["ilist"])[:lst["inum"]]].max())
+    lst.update(neighbors=np.ascontiguousarray(nb[:room].reshape(-1)), numneigh=num, maxneighs=room)
+    return lst
+
+
+def _with_room(lst, room):
+    stride, rows = lst["stride"], lst["maxneighs"]
+    nb = np.zeros((room, stride), np.int32)
+    nb[:rows] = np.asarray(lst["neighbors"]).reshape(rows, stride)
+    return dict(lst, neighbors=nb.reshape(-1), maxneighs=room)
+
+
+CASES = [("plain", 8, 0), ("plain", 4, 200), ("plain", 8, 430), ("plain", 4, 860),
+         ("plain", 8, 1400), ("half", 8, 0), ("half", 4, 230), ("half", 8, 480), ("half", 4, 980),
+         ("half", 8, 1600)]
+
+
+@pytest.mark.parametrize("scheme,precision,longest", CASES)
+def test_rows_not_room(gpu, scheme, precision, longest):
+    half = scheme == "half"
+    wl = systems.make_workload("eam_alloy_8k" if half else "lj_ghost_262k", cells=(4, 4, 5), seed=8)
+    sysm = systems.System(wl.x, wl.types, wl.box, wl.cutoff + wl.skin)
+    sysm.build_list(wl.cutoff + wl.skin, kind=harness.LIST_HALF if half else harness.LIST_FULL)
+    tight = _filled(sysm, wl.cutoff, longest)
+    model = ("eam", wl.tables) if half else ("lj", wl.lj)
+    forces = []
+    for lst in (tight, _with_room(tight, 2500)):
+        sysm.list = lst
+        pj = PairJax(sysm, model, precision=precision, accumulation=scheme)
+        print(f"rows not room {scheme} precision={precision} longest={tight['maxneighs']} "
+              f"room={lst['maxneighs']} nall={sysm.nall}", flush=True)
+        info = pj.compute()
+        forces.append(pj.forces().copy())
+    pos, sp = O.pack_atoms(sysm.x, sysm.type, sysm.nall, pj.max_atoms, precision)
+    s, r, m, count, _ = O.pack_neighbors(sysm.x, tight, max_atoms=pj.max_atoms,
+                                         max_edges=pj.max_edges, nlocal=sysm.nlocal,
+                                         cutoff=wl.cutoff)
+    kw = dict(nlocal=sysm.nlocal, nghost=sysm.nghost, senders=s, receivers=r, mask=m,
+              precision=precision)
+    if half:
+        ref = O.eam_compute(wl.tables, pos, sp, ghost_owner=sysm.ghost_owner, mode=O.HALF, **kw)
+    else:
+        ref = O.lj_compute(wl.lj, pos, mode=O.PLAIN, **kw)
+    assert info.edge_count == count
+    assert_energy(precision, info.energy, ref["energy"], sysm.nlocal)
+    assert_forces(precision, forces[0][:sysm.nall], ref["forces"][:sysm.nall])
+    assert np.array_equal(forces[0], forces[1])
