@@ -122,13 +122,17 @@ int ensure_incidence(Handle &h, long entries = 0)
   if (!h.d_deg) {
     fresh = true;
     const long chunks = (A + 1 + 4095) / 4096;
+    // d_deg last: it says that all of them are there (an earlier failure keeps what it got)
+    auto get = [&](auto **p, long n) { return *p ? hipSuccess : dalloc(p, n); };
+    auto get_scalars = [&](void **p) { return *p ? hipSuccess : hipMalloc(p, A * h.scalar_bytes()); };
+    if ((e = get(&h.d_inc_loc, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence offsets)");
+    if ((e = get(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
+    if ((e = get(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
+    if ((e = get(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");
+    if ((e = get(&h.d_bins, lk::bin_words(A))) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bins)");
+    if ((e = get_scalars(&h.d_rho_part)) != hipSuccess) return hip_fail(h, e, "hipMalloc(rho partials)");
+    if ((e = get_scalars(&h.d_epair)) != hipSuccess) return hip_fail(h, e, "hipMalloc(pair energy)");
     if ((e = dalloc(&h.d_deg, A + 2)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence counts)");
-    if ((e = dalloc(&h.d_inc_loc, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence offsets)");
-    if ((e = dalloc(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
-    if ((e = dalloc(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
-    if ((e = dalloc(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");
-    if ((e = hipMalloc(&h.d_rho_part, A * h.scalar_bytes())) != hipSuccess) return hip_fail(h, e, "hipMalloc(rho partials)");
-    if ((e = hipMalloc(&h.d_epair, A * h.scalar_bytes())) != hipSuccess) return hip_fail(h, e, "hipMalloc(pair energy)");
     if ((e = hipMemset(h.d_deg, 0, sizeof(int) * (A + 2))) != hipSuccess) return hip_fail(h, e, "hipMemset(incidence counts)");
   }
   const long need = entries > 2L * h.contract.max_edges ? entries : 2L * h.contract.max_edges;

@@ -50,6 +50,13 @@ struct FusedPack {
 // List-built incidence entries on their way hold atom and place in 32 bits up to this many atoms,
 // in 64 past it.
 constexpr long kBinAtoms32 = (1L << 26) - 1;
+// The build's bins hold 1 << kBinMinLog atoms at least; its working words for a capacity of atoms:
+// four counters and offsets per bin, one more offset and the longest row.
+constexpr int kBinMinLog = 2;
+constexpr long bin_words(long atoms)
+{
+  return 4 * ((atoms + (1 << kBinMinLog) - 1) >> kBinMinLog) + 2;
+}
 
 struct Handle {
   lk_contract contract{};
@@ -158,8 +165,7 @@ struct Handle {
   bool list_bits_filter = true;    // list-built incidence filtered by the pack's validity bits
   long inc_cap = 0;               // capacity of d_inc_tmp / d_inc (entries)
   // list-built incidence lists: the bins' counts and offsets and the list row of each atom
-  int *d_bins = nullptr;        // [bins_cap]
-  long bins_cap = 0;
+  int *d_bins = nullptr;        // [bin_words(max_atoms)]
   int *d_row_of = nullptr;      // [max_atoms]
   // the neighbour list of the last lk_pack_edges: the two-sided incidence lists are built from
   // its slots once per list (lk_set_list_epoch) and filtered each step by the pack's bits

@@ -305,7 +305,6 @@ constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 // of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
 constexpr int kBinLog = 6;
 constexpr int kBinAtoms = 1 << kBinLog;  // at most
-constexpr int kBinLeastLog = 2;
 constexpr int kBinPool = 62 * 1024;      // LDS of a bin's lists (two blocks or more share a CU)
 constexpr int kBinWaves = 16;            // waves of a counting block: kBinWaves / W 64-row tiles
 constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
@@ -324,7 +323,7 @@ __host__ __device__ inline BinLayout bin_layout(long longest, bool fold)
   const long per = fold ? (longest * 5 / 4 + 7) / 4 * 4 : (longest + 7) / 4 * 4;
   const long pitch = longest | 1;
   BinLayout y{kBinLog, 0, 0};
-  while (y.bin_log > kBinLeastLog && (4 * (per + pitch)) << y.bin_log > kBinPool) --y.bin_log;
+  while (y.bin_log > kBinMinLog && (4 * (per + pitch)) << y.bin_log > kBinPool) --y.bin_log;
   if ((4 * (per + pitch)) << y.bin_log <= kBinPool) {
     y.per_atom = static_cast<int>(per);
     y.pitch = static_cast<int>(pitch);
@@ -1649,15 +1648,6 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   L.layout = bin_layout(L.maxneighs, fold);
   Bins B;
   B.cap = (atoms + (1 << L.layout.bin_log) - 1) >> L.layout.bin_log;
-  const long words = 4L * B.cap + 2;
-  if (words > h.bins_cap) {  // rarely: a list with more room; a build may be running
-    if (hipError_t e = hipDeviceSynchronize(); e != hipSuccess) return e;
-    if (h.d_bins) (void)hipFree(h.d_bins);
-    h.d_bins = nullptr;
-    h.bins_cap = 0;
-    if (hipError_t e = hipMalloc(&h.d_bins, words * sizeof(int)); e != hipSuccess) return e;
-    h.bins_cap = words;
-  }
   B.next = h.d_bins;
   B.out = B.next + B.cap;
   B.off = B.out + B.cap;
@@ -1724,6 +1714,33 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   else
     finish(reinterpret_cast<uint64_t *>(h.d_inc_tmp));
   return hipGetLastError();
+}
+
+// The incidence lists of the neighbour list, built once per list: by the engine's epoch (or every
+// step when it gives none) and the list's shape. A build that failed leaves no lists to reuse.
+static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold)
+{
+  Handle::IncKey key;
+  key.epoch = h.list_epoch;
+  key.ilist = h.list_ilist;
+  key.neighbors = h.list_neighbors;
+  key.stride = h.list_stride;
+  key.rows = h.list_rows;
+  key.maxneighs = h.list_maxneighs;
+  key.half_filter = h.list_half_filter;
+  key.fold = fold ? 1 : 0;
+  if (h.list_epoch >= 0 && key == h.inc_key) return hipSuccess;
+  h.inc_key = Handle::IncKey{};
+  const hipError_t e = build_incidence_from_list(h, s, fold);
+  if (e == hipSuccess) h.inc_key = key;
+  return e;
+}
+
+// The incidence lists of the packed edges, built every step.
+static hipError_t lists_of_edges(Handle &h, hipStream_t s, int nall)
+{
+  h.inc_key = Handle::IncKey{};  // no list's any more
+  return build_incidence(h, s, nall);
 }
 
 // The sweeps' filter: none for lists built from packed edges or from a matrix, whose slots the
@@ -2210,22 +2227,9 @@ hipError_t launch_edge_force(Handle &h, hipStream_t s, int nlocal, int nghost, i
                : lj_edge_force<float>(h, s, nlocal, nghost, flags, scale, f, x);
   hipError_t e = hipSuccess;
   if (from_list) {
-    Handle::IncKey key;
-    key.epoch = h.list_epoch;
-    key.ilist = h.list_ilist;
-    key.neighbors = h.list_neighbors;
-    key.stride = h.list_stride;
-    key.rows = h.list_rows;
-    key.maxneighs = h.list_maxneighs;
-    key.half_filter = h.list_half_filter;
-    key.fold = 0;  // the edge-force sweeps walk whole lists
-    if (h.list_epoch < 0 || !(key == h.inc_key)) {
-      e = build_incidence_from_list(h, s, false);
-      h.inc_key = key;
-    }
+    e = lists_of_list(h, s, false);  // the edge-force sweeps walk whole lists
   } else {
-    e = build_incidence(h, s, nlocal + nghost);
-    h.inc_key = Handle::IncKey{};
+    e = lists_of_edges(h, s, nlocal + nghost);
   }
   if (e != hipSuccess) return e;
   return f64 ? eam_edge_force<double>(h, s, nlocal, nghost, flags, scale, f, x, from_list)
@@ -2240,23 +2244,9 @@ hipError_t launch_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost, in
   if (phase == kPhaseForce) {
     // the incidence lists are the ones this step's density pass used
   } else if (from_list) {
-    // once per list: the engine's epoch (or every step when it gives none) and the list's shape
-    Handle::IncKey key;
-    key.epoch = h.list_epoch;
-    key.ilist = h.list_ilist;
-    key.neighbors = h.list_neighbors;
-    key.stride = h.list_stride;
-    key.rows = h.list_rows;
-    key.maxneighs = h.list_maxneighs;
-    key.half_filter = h.list_half_filter;
-    key.fold = h.accum == LK_ACCUM_PLAIN ? 1 : 0;
-    if (h.list_epoch < 0 || !(key == h.inc_key)) {
-      e = build_incidence_from_list(h, s, key.fold != 0);
-      h.inc_key = key;
-    }
+    e = lists_of_list(h, s, h.accum == LK_ACCUM_PLAIN);
   } else {
-    e = build_incidence(h, s, nlocal + nghost);
-    h.inc_key = Handle::IncKey{};  // the entries are edge-built now
+    e = lists_of_edges(h, s, nlocal + nghost);
   }
   if (e != hipSuccess) return e;
   const bool f64 = h.contract.precision == LK_FLOAT64;
