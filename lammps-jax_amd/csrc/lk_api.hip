@@ -57,11 +57,11 @@ void free_all(Handle &h)
                   h.d_tile_off,  h.d_bits,      h.d_fp,          h.d_rho,       h.d_partials,
                   h.d_result,    h.d_ghost_owner, h.d_ghost_off, h.d_ghost_list, h.d_done,
                   h.d_deg,       h.d_inc_loc,   h.d_inc_part,    h.d_inc_tmp,   h.d_inc,
-                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,
+                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,      h.d_inc_bit,
                   h.d_matrix,    h.d_num_neighbors, h.d_identity, h.d_inc_len,
                   h.tl.keys,     h.tl.keys_sorted, h.tl.rows_in, h.tl.order,  h.tl.sort_tmp,
                   h.tl.atom,     h.tl.nn,       h.tl.uni,        h.tl.ucount,   h.tl.lid,
-                  h.tl.box,      h.d_row_of,    h.d_rowmark,   h.d_nonrow,      h.d_htab,      h.tl.ustat, h.d_dtab};
+                  h.tl.box,      h.d_rowmark,   h.d_nonrow,      h.d_htab,      h.tl.ustat, h.d_dtab};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (h.h_result) (void)hipHostFree(h.h_result);
@@ -128,7 +128,6 @@ int ensure_incidence(Handle &h, long entries = 0)
     if ((e = get(&h.d_inc_loc, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence offsets)");
     if ((e = get(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
     if ((e = get(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
-    if ((e = get(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");
     if ((e = get(&h.d_bins, lk::bin_words(A))) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bins)");
     if ((e = get_scalars(&h.d_rho_part)) != hipSuccess) return hip_fail(h, e, "hipMalloc(rho partials)");
     if ((e = get_scalars(&h.d_epair)) != hipSuccess) return hip_fail(h, e, "hipMalloc(pair energy)");
@@ -147,14 +146,18 @@ int ensure_incidence(Handle &h, long entries = 0)
                 "fit in int)");
   if (need > h.inc_cap) {
     if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(h, e, "hipDeviceSynchronize");
-    for (void *p : {static_cast<void *>(h.d_inc_tmp), static_cast<void *>(h.d_inc)})
+    for (void *p : {static_cast<void *>(h.d_inc_tmp), static_cast<void *>(h.d_inc),
+                    static_cast<void *>(h.d_inc_bit)})
       if (p) (void)hipFree(p);
     h.d_inc_tmp = nullptr;
     h.d_inc = nullptr;
+    h.d_inc_bit = nullptr;
     h.inc_cap = 0;
     const long words = h.contract.max_atoms <= lk::kBinAtoms32 ? need : need + (need + 1) / 2;
     if ((e = dalloc(&h.d_inc_tmp, words)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence staging)");
     if ((e = dalloc(&h.d_inc, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lists)");
+    if (h.scalar_bytes() == 4 && h.list_bits_filter)
+      if ((e = dalloc(&h.d_inc_bit, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bits)");
     h.inc_cap = need;
     h.inc_key = Handle::IncKey{};  // rebuild
     fresh = true;
@@ -700,6 +703,7 @@ int lk_pack_edges(lk_handle *w, void *stream, const double *x, const int *ilist,
                                        nlocal, duplicate, half_filter, unique);
   if (e == hipSuccess && h.nonrow_blocks > 0)
     e = lk::launch_mark_rows(h, as_stream(stream), ilist, static_cast<int>(rows), nlocal);
+  if (e == hipSuccess) e = lk::launch_list_bits(h, as_stream(stream));
   if (e != hipSuccess) return hip_fail(h, e, "pack_edges");
   h.result_mirrored = false;
   return LK_OK;

@@ -162,11 +162,14 @@ struct Handle {
   int *d_identity = nullptr;       // row i is atom i
   bool matrix_copied = false;
   long matrix_epoch = -2;          // list epoch of the last copy
-  bool list_bits_filter = true;    // list-built incidence filtered by the pack's validity bits
-  long inc_cap = 0;               // capacity of d_inc_tmp / d_inc (entries)
-  // list-built incidence lists: the bins' counts and offsets and the list row of each atom
+  bool list_bits_filter = true;    // list-built entries filtered as the pack filters their slots
+  long inc_cap = 0;               // capacity of d_inc_tmp / d_inc / d_inc_bit (entries)
+  // list-built incidence lists: the bins' counts and offsets
   int *d_bins = nullptr;        // [bin_words(max_atoms)]
-  int *d_row_of = nullptr;      // [max_atoms]
+  // float32: each list-built entry's place among the validity bits, written for sweeps that follow
+  // a pack called on its own (inc_bits: those of the lists that stand)
+  uint32_t *d_inc_bit = nullptr;  // [inc_cap]
+  bool inc_bits = false;
   // the neighbour list of the last lk_pack_edges: the two-sided incidence lists are built from
   // its slots once per list (lk_set_list_epoch) and filtered each step by the pack's bits
   const int *list_ilist = nullptr;
@@ -279,6 +282,7 @@ hipError_t launch_edge_force(Handle &h, hipStream_t s, int nlocal, int nghost, i
 hipError_t launch_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost, int flags,
                             double scale, double *f, const double *x, bool from_list,
                             const FusedPack &pack = FusedPack{}, int phase = kPhaseAll);
+hipError_t launch_list_bits(Handle &h, hipStream_t s);
 
 // LAMMPS comm buffers for model rows (lk_comm.hip): `slots` doubles per buffer row.
 int comm_slots(const Handle &h, int width);

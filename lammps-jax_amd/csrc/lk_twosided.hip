@@ -253,7 +253,6 @@ struct ListArgs {
   int max_atoms;
   int half_filter;
   int *out_n;   // list slots of each atom's row (0: the atom is no row)
-  int *row_of;  // list row of each atom (-1: none)
   int *loc;     // first entry of each atom
   int *part;    // zero (loc holds whole offsets)
   int *len;     // entries of each atom
@@ -366,10 +365,7 @@ struct Bins {
 __global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < L.max_atoms) {
-    L.out_n[i] = 0;
-    L.row_of[i] = -1;
-  }
+  if (i < L.max_atoms) L.out_n[i] = 0;
   if (i < B.cap) {
     B.next[i] = 0;
     B.out[i] = 0;
@@ -377,7 +373,7 @@ __global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
   if (i < (L.max_atoms + kScanChunk) / kScanChunk) L.part[i] = 0;
 }
 
-// Count (SCATTER false: the in- and out-entries of each bin; also out_n and row_of) and scatter.
+// Count (SCATTER false: the in- and out-entries of each bin; also out_n) and scatter.
 // One lane per row, the W waves of a tile sharing its slots; entries of adjacent lanes in the same
 // bin (adjacent rows' k-th neighbours mostly are) count as one run, so a wave does one LDS update
 // per run.
@@ -415,7 +411,6 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   };
   if (!SCATTER && wq == 0 && i >= 0) {
     L.out_n[i] = nn;
-    L.row_of[i] = ii;
     const int q = slot_of(i >> bin_log);
     atomicAdd(q >= 0 ? &aux[q] : &B.out[i >> bin_log], nn);
   }
@@ -930,6 +925,50 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
   }
 }
 
+// The place of each list entry's slot among the pack's validity bits (word (jj >> 5) * pitch + ii, bit
+// jj & 31, the words of a row `pitch` apart), for float32 sweeps after a pack called on its own:
+// one block per 64-row tile, the waves sharing its slots out in ranges. An out-entry's place follows
+// from the kept slots before it, an in-entry is found by bisection in the list of the atom its slot
+// names (out-entries come first, without the side bit, so the whole list is in order against the
+// key); the folded ones are not there, and equal ones stand for equal slots. Once per list and only
+// for such calls (46 us at 62,500 atoms of a half list). A search of the sender's row in the sweeps,
+// for every entry near the cutoff, read the engine's list on every step and, with a neighbour shell
+// on the cutoff, took 46.6 us of that box's density sweep and 56.8 of its force sweep, now 16.0 and
+// 29.6.
+constexpr int kBitWaves = 16;
+
+__global__ __launch_bounds__(kBitWaves *kWave) LK_EIGHT_WAVES
+void k_inc_bits(ListArgs L, int pitch, uint32_t *__restrict__ inc_bit)
+{
+  __shared__ int kept[kBitWaves][kWave];
+  const int wave = wave_in_block(), lane = threadIdx.x & (kWave - 1);
+  const int ii = blockIdx.x * kWave + lane;
+  int nn = 0, i = -1;
+  if (ii < L.rows) i = list_row(L, ii, nn);
+  const int nmax = wave_max_int(nn), per = (nmax + kBitWaves - 1) / kBitWaves;
+  const int j0 = min(wave * per, nn), j1 = min(j0 + per, nn);
+  int c = 0;
+  for (int jj = j0; jj < j1; ++jj) {
+    int j;
+    c += list_neighbor(L, i, jj, j) ? 1 : 0;
+  }
+  kept[wave][lane] = c;
+  __syncthreads();
+  int at = i >= 0 ? L.loc[i] : 0;
+  for (int w = 0; w < wave; ++w) at += kept[w][lane];
+  for (int jj = j0; jj < j1; ++jj) {
+    int j;
+    if (!list_neighbor(L, i, jj, j)) continue;
+    const uint32_t bit = ((static_cast<uint32_t>(jj >> 5) * static_cast<uint32_t>(pitch) +
+                           static_cast<uint32_t>(ii)) << 5) | static_cast<uint32_t>(jj & 31);
+    inc_bit[at++] = bit;
+    const uint32_t *list = reinterpret_cast<const uint32_t *>(L.inc) + L.loc[j];
+    const uint32_t key = static_cast<uint32_t>(i) | (1u << 31);
+    const int n = L.len[j];
+    for (int q = lower_bound(list, n, key); q < n && list[q] == key; ++q) inc_bit[L.loc[j] + q] = bit;
+  }
+}
+
 template <int G, typename T>
 __device__ __forceinline__ T group_sum(T v)
 {
@@ -953,11 +992,8 @@ struct TwoSided {
   const int *ghost_off;
   const int *ghost_list;
   int nblk;             // 64-atom partial tiles over nall
-  const uint32_t *bits;     // kFromBits: the pack's validity bits by list row, and the list
-  const int *row_of, *out_n;  // each atom's list row and its slots
-  const int *neighbors;
-  long stride;
-  int max_atoms;
+  const uint32_t *bits;     // kFromBits: the pack's validity bits
+  const uint32_t *inc_bit;  // kFromBits: each entry's place in them (k_inc_bits)
   double cutsq_pack;        // the pack's filter: rsq <= cutsq in float64 (cpp:91)
   float cutsq_lo, cutsq_hi; // cutsq_pack rounded down and up to float
   const int *ghost_flag;    // 1 when a packed edge starts on a ghost row (the pack's flag)
@@ -978,8 +1014,8 @@ struct TwoSided {
 // computed in float, exceeds twice that bound and at least 8u r2, which covers the rounding of
 // r2 +- band against cutsq rounded down (up) to float. Only an r2 inside the band looks further:
 // where the pack ran in this call it forms rsq from the engine's positions as the pack did (the
-// sign of the differences does not matter), else it finds the entry's slot in its sender's row and
-// reads that slot's validity bit. Per row, BandRow bounds the band of every entry the model's cutoff lets through (l1 <= sqrt(3)
+// sign of the differences does not matter), else it reads the validity bit of the entry's slot. Per
+// row, BandRow bounds the band of every entry the model's cutoff lets through (l1 <= sqrt(3)
 // rc_model, and the neighbour's 1-norm <= the row's + l1), so most entries are decided by one
 // comparison with a row threshold. Lists built from packed edges hold kept slots only (no
 // filter).
@@ -1011,9 +1047,9 @@ __device__ __forceinline__ BandRow<S> band_row(const TwoSided &t, const Atom4<S>
 // kernel held 94 SGPRs in the float32 density sweep: one block per CU, 59 -> 71 us at 256,000 atoms.)
 enum Filter { kAllKept = 0, kFromX = 1, kFromBits = 2 };
 
-// The decision inside the band: atom a's entry with atom o, on o's row when `in`.
+// The decision inside the band: entry q of atom a's list, with atom o.
 template <int FILTER>
-__device__ __forceinline__ bool kept_by_pack(const TwoSided &t, int a, int o, bool in)
+__device__ __forceinline__ bool kept_by_pack(const TwoSided &t, int a, int o, int q)
 {
   if constexpr (FILTER == kFromX) {
 #pragma clang fp contract(off)
@@ -1025,23 +1061,20 @@ __device__ __forceinline__ bool kept_by_pack(const TwoSided &t, int a, int o, bo
     }
     return !(rsq > t.cutsq_pack);
   } else {
-    const int snd = in ? o : a, rcv = in ? a : o;
-    const int ii = t.row_of[snd], nn = t.out_n[snd];
-    for (int jj = 0; jj < nn; ++jj)
-      if ((t.neighbors[static_cast<long>(jj) * t.stride + snd] & kNeighMask) == rcv)
-        return ((t.bits[static_cast<long>(jj >> 5) * t.max_atoms + ii] >> (jj & 31)) & 1u) != 0;
-    return false;
+    const uint32_t at = t.inc_bit[q];
+    return ((t.bits[at >> 5] >> (at & 31u)) & 1u) != 0;
   }
 }
 
 template <int FILTER, typename S>
-__device__ __forceinline__ bool slot_kept(const TwoSided &t, int a, uint32_t v, S r2, S dx, S dy,
-                                          S dz, const BandRow<S> &br, const Atom4<S> &xo)
+__device__ __forceinline__ bool slot_kept(const TwoSided &t, int a, uint32_t v, int q, S r2, S dx,
+                                          S dy, S dz, const BandRow<S> &br, const Atom4<S> &xo)
 {
   if constexpr (FILTER == kAllKept) return true;
   if constexpr (sizeof(S) == 8) {
     (void)a;
     (void)v;
+    (void)q;
     (void)dx;
     (void)dy;
     (void)dz;
@@ -1057,7 +1090,7 @@ __device__ __forceinline__ bool slot_kept(const TwoSided &t, int a, uint32_t v, 
     const float band = 2.0f * u * (s * (2.0f * l1 + u * s) + 4.0f * r2);
     if (r2 + band <= t.cutsq_lo) return true;
     if (r2 - band > t.cutsq_hi) return false;
-    return kept_by_pack<FILTER>(t, a, static_cast<int>(v & kIncAtom), (v >> 31) != 0);
+    return kept_by_pack<FILTER>(t, a, static_cast<int>(v & kIncAtom), q);
   }
 }
 
@@ -1133,13 +1166,13 @@ void k_eam_density_inc(EamArgs<S> m, TwoSided t, S *__restrict__ rho_part, S *__
       // Two entries per lane at a time (k and k + G): both entries load together, then both
       // records, so a pair of entries costs two memory round trips; a skipped or missing entry
       // gathers the row's own record.
-      auto dens = [&](uint32_t v, const Atom4<S> &xo) {
+      auto dens = [&](uint32_t v, int q, const Atom4<S> &xo) {
         const bool in = (v >> 31) != 0;
         if (!HALF && in) return;  // plain: density and pair energy stay on the sender
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 < m.cutsq)) return;
-        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, q, r2, dx, dy, dz, br, xo)) return;
         const S rinv = rsqrt_nr(r2);
         const S rr = r2 * rinv;
         const Locator<S> L2 = locate_mul(rr, m.inv_dr, m.nr);
@@ -1166,8 +1199,8 @@ void k_eam_density_inc(EamArgs<S> m, TwoSided t, S *__restrict__ rho_part, S *__
         const bool s1 = !HALF && (v1 >> 31) != 0, s2 = !two || (!HALF && (v2 >> 31) != 0);
         const Atom4<S> x1 = m.atoms[s1 ? a : static_cast<int>(v1 & kIncAtom)];
         const Atom4<S> x2 = m.atoms[s2 ? a : static_cast<int>(v2 & kIncAtom)];
-        dens(v1, x1);
-        if (two) dens(v2, x2);
+        dens(v1, q1, x1);
+        if (two) dens(v2, q2, x2);
       }
     }
     rho = group_sum<G>(rho);
@@ -1315,13 +1348,15 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
       // is skipped, so no branch surrounds a load).
       struct Gathered {
         uint32_t v;
+        int q;  // the entry's index
         bool skip;
         Atom4<S> xo;
         S fpo;
       };
-      auto gather = [&](uint32_t v, bool present) -> Gathered {
+      auto gather = [&](uint32_t v, int q, bool present) -> Gathered {
         Gathered e;
         e.v = v;
+        e.q = q;
         const bool in = (v >> 31) != 0;
         const int o = static_cast<int>(v & kIncAtom);
         // plain: an uncounted sender gives no gradient; a folded pair counts each counted end
@@ -1344,7 +1379,7 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 < m.cutsq)) return;
-        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, e.q, r2, dx, dy, dz, br, xo)) return;
         const S rinv = rsqrt_nr(r2);
         const S rr = r2 * rinv;
         const Locator<S> L2 = locate_mul(rr, m.inv_dr, m.nr);
@@ -1422,7 +1457,7 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
       if constexpr (sizeof(S) == 8) {
         IncCursor<G> cur(t, b, L, gl);
         for (int k = gl; k < L; k += G) {
-          const Gathered e = gather(cur.v, true);
+          const Gathered e = gather(cur.v, 0, true);  // float64 needs no index
           cur.advance(t, k);
           edge(e);
         }
@@ -1432,8 +1467,8 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
         uint32_t v1 = static_cast<uint32_t>(t.inc[q1]);
         uint32_t v2 = static_cast<uint32_t>(t.inc[q2]);
         for (int k = gl; k < L; k += 2 * G) {
-          const Gathered e1 = gather(v1, true);
-          const Gathered e2 = gather(v2, k + G < L);
+          const Gathered e1 = gather(v1, q1, true);
+          const Gathered e2 = gather(v2, q2, k + G < L);
           asm volatile("" ::: "memory");  // keep the next entries' loads behind the gathers
           q1 = min(b + k + 2 * G, last);
           q2 = min(b + k + 3 * G, last);
@@ -1525,12 +1560,12 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
         const int co = static_cast<int>(v & kIncAtom) < erows ? 1 : 0;
         return (in ? 0 : (a < erows ? 1 : 0)) + ((in || (v & kIncPaired)) ? co : 0);
       };
-      auto pair = [&](uint32_t v, int w, const Atom4<S> &xo) {
+      auto pair = [&](uint32_t v, int q, int w, const Atom4<S> &xo) {
         if (w == 0) return;
         S dx, dy, dz;
         const S r2 = geometry(xa, xo, dx, dy, dz);
         if (!(r2 > tiny && r2 < m.cutsq)) return;  // export_model.py:22
-        if (!slot_kept<FILTER>(t, a, v, r2, dx, dy, dz, br, xo)) return;
+        if (!slot_kept<FILTER>(t, a, v, q, r2, dx, dy, dz, br, xo)) return;
         const S inv_r2 = m.sigsq / r2;
         const S inv_r6 = inv_r2 * inv_r2 * inv_r2;
         if (!(v >> 31)) en += m.edge_scale * (m.four_eps * (inv_r6 * inv_r6 - inv_r6));
@@ -1550,8 +1585,8 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
         const int w1 = ends(v1), w2 = two ? ends(v2) : 0;
         const Atom4<S> x1 = m.atoms[w1 ? static_cast<int>(v1 & kIncAtom) : a];
         const Atom4<S> x2 = m.atoms[w2 ? static_cast<int>(v2 & kIncAtom) : a];
-        pair(v1, w1, x1);
-        pair(v2, w2, x2);
+        pair(v1, q1, w1, x1);
+        pair(v2, q2, w2, x2);
       }
     }
     en = group_sum<G>(en);
@@ -1626,9 +1661,9 @@ static hipError_t build_incidence(Handle &h, hipStream_t s, int nall)
   return hipGetLastError();
 }
 
-static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
+static ListArgs list_args(Handle &h, bool fold)
 {
-  ListArgs L;
+  ListArgs L{};
   L.ilist = h.list_ilist;
   L.numneigh = h.list_numneigh;
   L.neighbors = h.list_neighbors;
@@ -1638,14 +1673,19 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   L.max_atoms = h.contract.max_atoms;
   L.half_filter = h.list_half_filter;
   L.out_n = h.d_deg;
-  L.row_of = h.d_row_of;
   L.loc = h.d_inc_loc;
   L.part = h.d_inc_part;
   L.len = h.d_inc_len;
   L.inc = h.d_inc;
-  const int atoms = L.max_atoms;
   L.fold = fold ? 1 : 0;
   L.layout = bin_layout(L.maxneighs, fold);
+  return L;
+}
+
+static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
+{
+  ListArgs L = list_args(h, fold);
+  const int atoms = L.max_atoms;
   Bins B;
   B.cap = (atoms + (1 << L.layout.bin_log) - 1) >> L.layout.bin_log;
   B.next = h.d_bins;
@@ -1716,9 +1756,7 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   return hipGetLastError();
 }
 
-// The incidence lists of the neighbour list, built once per list: by the engine's epoch (or every
-// step when it gives none) and the list's shape. A build that failed leaves no lists to reuse.
-static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold)
+static Handle::IncKey list_key(const Handle &h, bool fold)
 {
   Handle::IncKey key;
   key.epoch = h.list_epoch;
@@ -1729,11 +1767,43 @@ static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold)
   key.maxneighs = h.list_maxneighs;
   key.half_filter = h.list_half_filter;
   key.fold = fold ? 1 : 0;
+  return key;
+}
+
+// The incidence lists of the neighbour list, built once per list: by the engine's epoch (or every
+// step when it gives none) and the list's shape. A build that failed leaves no lists to reuse.
+static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold)
+{
+  const Handle::IncKey key = list_key(h, fold);
   if (h.list_epoch >= 0 && key == h.inc_key) return hipSuccess;
   h.inc_key = Handle::IncKey{};
+  h.inc_bits = false;
   const hipError_t e = build_incidence_from_list(h, s, fold);
   if (e == hipSuccess) h.inc_key = key;
   return e;
+}
+
+// The places of the lists' entries among the validity bits, for the sweeps that read them.
+static hipError_t bits_of_list(Handle &h, hipStream_t s)
+{
+  if (h.inc_bits || !h.d_inc_bit) return hipSuccess;
+  const ListArgs L = list_args(h, h.inc_key.fold != 0);
+  const int tiles = (L.rows + kWave - 1) / kWave;
+  StageTimer timer(h, s, "inc_bits");
+  if (tiles > 0)
+    hipLaunchKernelGGL(k_inc_bits, dim3(tiles), dim3(kBitWaves * kWave), 0, s, L,
+                       h.contract.max_atoms, h.d_inc_bit);
+  const hipError_t e = hipGetLastError();
+  h.inc_bits = e == hipSuccess;
+  return e;
+}
+
+// A pack called on its own over the list that the incidence lists already stand for: what its sweeps
+// will need of the list is read here, so that they read no list on a step that rebuilds none.
+hipError_t launch_list_bits(Handle &h, hipStream_t s)
+{
+  if (h.list_epoch < 0 || !(list_key(h, h.inc_key.fold != 0) == h.inc_key)) return hipSuccess;
+  return bits_of_list(h, s);
 }
 
 // The incidence lists of the packed edges, built every step.
@@ -1781,11 +1851,7 @@ static TwoSided two_sided_args(Handle &h, int nlocal, int nghost, const double *
   t.ghost_list = h.d_ghost_list;
   t.nblk = (t.nall + kRowAtoms - 1) / kRowAtoms;
   t.bits = h.d_bits;
-  t.row_of = h.d_row_of;
-  t.out_n = h.d_deg;
-  t.neighbors = h.inc_key.neighbors;
-  t.stride = h.inc_key.stride;
-  t.max_atoms = h.contract.max_atoms;
+  t.inc_bit = h.d_inc_bit;
   t.cutsq_pack = h.contract.cutoff * h.contract.cutoff;
   t.cutsq_lo = static_cast<float>(t.cutsq_pack);
   t.cutsq_hi = t.cutsq_lo;
@@ -2228,6 +2294,7 @@ hipError_t launch_edge_force(Handle &h, hipStream_t s, int nlocal, int nghost, i
   hipError_t e = hipSuccess;
   if (from_list) {
     e = lists_of_list(h, s, false);  // the edge-force sweeps walk whole lists
+    if (e == hipSuccess && sweep_filter(h, true, FusedPack{}) == kFromBits) e = bits_of_list(h, s);
   } else {
     e = lists_of_edges(h, s, nlocal + nghost);
   }
@@ -2245,6 +2312,7 @@ hipError_t launch_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost, in
     // the incidence lists are the ones this step's density pass used
   } else if (from_list) {
     e = lists_of_list(h, s, h.accum == LK_ACCUM_PLAIN);
+    if (e == hipSuccess && sweep_filter(h, true, pack) == kFromBits) e = bits_of_list(h, s);
   } else {
     e = lists_of_edges(h, s, nlocal + nghost);
   }
