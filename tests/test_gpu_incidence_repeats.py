@@ -26,7 +26,7 @@ def _far(x, xi, cutoff):
     return np.flatnonzero(np.sum((x - xi) ** 2, axis=1) > (cutoff + 0.1) ** 2)
 
 
-def _repeating(sysm, wl, longest, hubs):
+def _repeating(sysm, cutoff, longest, hubs):
     """The system's list with repeated entries (and far ones, see above)."""
     rng = np.random.default_rng(17)
     lst = dict(sysm.list)
@@ -43,9 +43,9 @@ def _repeating(sysm, wl, longest, hubs):
         if j in rows and i in rows[j] and rng.random() < 0.5:
             rows[j].insert(int(rng.integers(0, len(rows[j]) + 1)), i)
     for n, i in enumerate(owned):
-        rows[i] += _far(x[:hubs], x[i], wl.cutoff).tolist()
+        rows[i] += _far(x[:hubs], x[i], cutoff).tolist()
         if n % 3 == 0 and len(rows[i]) < longest:
-            rows[i] = np.resize(_far(x, x[i], wl.cutoff), longest - len(rows[i])).tolist() + rows[i]
+            rows[i] = np.resize(_far(x, x[i], cutoff), longest - len(rows[i])).tolist() + rows[i]
     room = max(len(r) for r in rows.values())
     nb = np.zeros((room, stride), np.int32)
     for i, r in rows.items():
@@ -68,27 +68,22 @@ CASES = [  # scheme, precision, cells, longest row, hubs
 ]
 
 
-@pytest.mark.parametrize("scheme,precision,cells,longest,hubs", CASES)
-def test_repeated_entries(gpu, scheme, precision, cells, longest, hubs):
+def _check(sysm, wl_cutoff, lst, model, scheme, precision, max_atoms=None):
     half = scheme == "half"
-    wl = systems.make_workload("eam_alloy_8k" if half else "lj_ghost_262k", cells=cells, seed=21)
-    sysm = systems.System(wl.x, wl.types, wl.box, wl.cutoff + wl.skin)
-    sysm.build_list(wl.cutoff + wl.skin, kind=harness.LIST_HALF if half else harness.LIST_FULL)
-    lst = _repeating(sysm, wl, longest, hubs)
-    model = ("eam", wl.tables) if half else ("lj", wl.lj)
-    pj = PairJax(sysm, model, precision=precision, accumulation=scheme)
-    print(f"repeated entries {scheme} precision={precision} cells={cells} "
-          f"room={lst['maxneighs']} hubs={hubs} nall={sysm.nall}", flush=True)
-    pos, sp = O.pack_atoms(sysm.x, sysm.type, sysm.nall, pj.max_atoms, precision)
-    s, r, m, count, _ = O.pack_neighbors(sysm.x, lst, max_atoms=pj.max_atoms,
+    pj = PairJax(sysm, model, precision=precision, accumulation=scheme, max_atoms=max_atoms,
+                 max_edges=128 * sysm.nall)
+    print(f"repeated entries {scheme} precision={precision} room={lst['maxneighs']} "
+          f"nall={sysm.nall} capacity={pj.max_atoms}", flush=True)
+    pos, sp = O.pack_atoms(sysm.x, sysm.type, sysm.nall, sysm.nall, precision)
+    s, r, m, count, _ = O.pack_neighbors(sysm.x, lst, max_atoms=sysm.nall,
                                          max_edges=pj.max_edges, nlocal=sysm.nlocal,
-                                         cutoff=wl.cutoff)
+                                         cutoff=wl_cutoff)
     kw = dict(nlocal=sysm.nlocal, nghost=sysm.nghost, senders=s, receivers=r, mask=m,
               precision=precision)
     if half:
-        ref = O.eam_compute(wl.tables, pos, sp, ghost_owner=sysm.ghost_owner, mode=O.HALF, **kw)
+        ref = O.eam_compute(model[1], pos, sp, ghost_owner=sysm.ghost_owner, mode=O.HALF, **kw)
     else:
-        ref = O.lj_compute(wl.lj, pos, mode=O.PLAIN, **kw)
+        ref = O.lj_compute(model[1], pos, mode=O.PLAIN, **kw)
     nall = sysm.nall
     first = None
     for fused in (True, True, True, False):
@@ -103,3 +98,34 @@ def test_repeated_entries(gpu, scheme, precision, cells, longest, hubs):
         assert info.energy == first[0] and np.array_equal(f, first[1])
         pj.list_epoch += 1  # the engine's rebuild signal: the same lists again
         pj.h.set_list_epoch(pj.list_epoch)
+
+
+@pytest.mark.parametrize("scheme,precision,cells,longest,hubs", CASES)
+def test_repeated_entries(gpu, scheme, precision, cells, longest, hubs):
+    half = scheme == "half"
+    wl = systems.make_workload("eam_alloy_8k" if half else "lj_ghost_262k", cells=cells, seed=21)
+    sysm = systems.System(wl.x, wl.types, wl.box, wl.cutoff + wl.skin)
+    sysm.build_list(wl.cutoff + wl.skin, kind=harness.LIST_HALF if half else harness.LIST_FULL)
+    lst = _repeating(sysm, wl.cutoff, longest, hubs)
+    _check(sysm, wl.cutoff, lst, ("eam", wl.tables) if half else ("lj", wl.lj), scheme, precision)
+
+
+@pytest.mark.parametrize("scheme,precision", [("plain", 4), ("plain", 8), ("half", 8)])
+def test_capacity_past_32_bit_entries(gpu, scheme, precision):
+    """A contract of more than 2^26 - 1 atoms, whose entries travel in 64 bits; rows of at most 32
+    slots, which is what such a capacity leaves of the validity bits' 27-bit addresses."""
+    half = scheme == "half"
+    a = 3.8 if half else 1.68
+    cutoff, skin = (3.5, 0.5) if half else (1.6, 0.2)
+    box = np.full(3, 6 * a)
+    rng = np.random.default_rng(2)
+    x = systems.fcc_lattice(6, 6, 6, a)
+    x = systems.wrap(x + rng.normal(0.0, 0.03 * a, size=x.shape), box)
+    types = rng.integers(1, 3, len(x)).astype(np.int32) if half else np.ones(len(x), np.int32)
+    sysm = systems.System(x, types, box, cutoff + skin)
+    sysm.build_list(cutoff + skin, kind=harness.LIST_HALF if half else harness.LIST_FULL)
+    lst = _repeating(sysm, cutoff, 0, 0)
+    assert lst["maxneighs"] <= 32, lst["maxneighs"]
+    model = (("eam", systems.synthetic_alloy_tables(cutoff=cutoff)) if half else
+             ("lj", dict(epsilon=1.0, sigma=1.0, cutoff=cutoff, edge_energy_scale=0.5)))
+    _check(sysm, cutoff, lst, model, scheme, precision, max_atoms=(1 << 26) + 1000)
