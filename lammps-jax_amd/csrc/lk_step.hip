@@ -805,11 +805,20 @@ static hipError_t step_onesided(Handle &h, hipStream_t s, const double *x, const
                            dim3(step_pack_grid<EAM>(groups, h.num_cus)), dim3(kStepWaves * kWave),
                            0, s, p, a, groups);
       };
-      // Sixteen waves per tile while the tiles fill two blocks per CU, eight past that: us by
-      // waves per tile 2, 4, 8, 16 (float32, packed edges; four were used at every size before)
+      // float32: sixteen waves per tile while the tiles fill two blocks per CU, eight past that; us by
+      // waves per tile 2, 4, 8, 16 (packed edges; four were used at every size before)
       //   16 tiles (1,008 atoms)  49, 33, 22, 17*   1,024 tiles (65,536)   68, 49, 41*, 45
       //   465 tiles (29,716)      58, 38, 28, 26*   2,048 tiles (131,072)  85, 75, 73*, 79
-      if (ntiles <= 2 * (h.num_cus > 0 ? h.num_cus : 256))
+      // float64, whose walk is one slot at a time and so waits longer for each: sixteen at every
+      // size; step in us by 8 and 16 (neighbour matrix; packed edges without a list epoch come
+      // within 1.5 us of it)
+      //   16 tiles (1,024 atoms)  46.7, 39.2*   1,024 tiles (65,536)    99.9, 98.7*
+      //   128 tiles (8,192)       48.5, 41.6*   1,088 tiles (69,632)   133.5, 124.4*
+      //   465 tiles (29,716)      61.2, 57.5*   2,048 tiles (131,072)  163.9, 159.3*
+      // (four waves of whole 32-slot words before: 98, 102, 113, 132, 166 and 169).
+      if constexpr (sizeof(S) == 8)
+        launch(std::integral_constant<int, 16>{});
+      else if (ntiles <= 2 * (h.num_cus > 0 ? h.num_cus : 256))
         launch(std::integral_constant<int, 16>{});
       else
         launch(std::integral_constant<int, 8>{});
