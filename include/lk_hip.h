@@ -6,13 +6,16 @@
  * sized once from the contract capacities (never resized), and the per-step results.
  *
  * Every entry point is stream-ordered on the caller's HIP stream (the Kokkos execution space
- * stream in a LAMMPS build); per step only lk_step_result synchronises. Work done once per
- * neighbour list may wait once: the two-sided schemes read one count back when they build the
- * incidence lists of a list over 4 M slots, and a working buffer that grows for a larger list
- * waits for the device before it is replaced. Pointers named x, f, ilist,
- * numneigh and neighbors are device pointers owned by the caller (the engine) and are never
- * freed here. Errors return a status code; lk_last_error gives the message. Nothing throws
- * across this boundary.
+ * stream in a LAMMPS build); per step only lk_step_result synchronises. A working buffer that
+ * grows for a larger neighbour list waits for the device before it is replaced; nothing else waits
+ * once per list. Pointers named x, f, ilist, numneigh and neighbors are device pointers owned by the
+ * caller (the engine) and are never freed here. A call reads the list it is given. The two-sided
+ * schemes also read the list of the last lk_pack_edges in the model call that follows it
+ * (lk_compute, lk_model_density) when that call builds the incidence lists: the first one of a list
+ * epoch, or every one without an epoch; until then ilist, numneigh and neighbors must stay as they
+ * were at the pack. lk_model_force reads no list. x (with the neighbour matrix also type) must stay
+ * as at the last pack until the model call that follows it. Errors return a status code; lk_last_error gives the message. Nothing throws across this
+ * boundary.
  *
  * Reference interfaces replaced (paths relative to the reference repository root):
  *   lk_create / lk_destroy   PairJaxKokkos::allocate_device_buffers (cpp/pair_jax_kokkos.cpp:355-398)
@@ -155,7 +158,7 @@ int lk_set_ghost_map(lk_handle *h, int nlocal, int nghost, const int *ghost_owne
  * that changes whenever it rebuilds the list (LAMMPS: the step of the last build, the same event
  * neighbor->ago == 0 marks in PairJaxKokkos::compute, cpp/pair_jax_kokkos.cpp:1010-1011). The
  * per-atom incidence lists are then built from the list slots once per list and filtered each
- * step by the pack's validity bits. -1 (the default): rebuilt at every compute.
+ * step as the pack filters the slots. -1 (the default): rebuilt at every compute.
  */
 int lk_set_list_epoch(lk_handle *h, long epoch);
 

@@ -147,8 +147,9 @@ struct Handle {
   int *d_inc_part = nullptr;    // [chunks] chunk offsets
   uint32_t *d_inc_tmp = nullptr;  // entries on their way into d_inc: [inc_cap] words, half as many
                                   // again past kBinAtoms32 atoms
-  int *d_inc = nullptr;         // [inc_cap] other atom | side << 31: all of an edge-built list's
-                                // entries in edge order, a list-built one's in-entries
+  int *d_inc = nullptr;         // [inc_cap] other atom | side << 31: an edge-built list's entries
+                                // in edge order; a list-built one's out-entries in slot order, then
+                                // its in-entries by row atom
   int *d_inc_len = nullptr;     // [max_atoms + 1] entries of each atom in d_inc
   void *d_rho_part = nullptr;   // [max_atoms] per-row density before the ghost fold
   void *d_epair = nullptr;      // [max_atoms] per-row pair energy

@@ -229,8 +229,9 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
       }
       return false;
     };
-    // The float32 and the pack-only kernels walk the slots jj0, jj0 + step, ... < jj1 two at a time: both entries are loaded one pair ahead, then both
-    // neighbour records gathered together, so a pair costs one memory round trip. Every load
+    // The float32 and the pack-only kernels walk the slots jj0, jj0 + step, ... < jj1 two at a
+    // time: both entries are loaded one pair ahead, then both neighbour records gathered
+    // together, so a pair costs one memory round trip. Every load
     // is unconditional (slots past the row read element 0 of the list and the record of atom 0,
     // which exist whenever the loop runs, and are unused), so the compiler counts them exactly
     // and waits for the gathers without waiting for the next pair's entries. The records are
@@ -328,7 +329,7 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
     // Each wave takes every W-th slot and ORs its bits into the tile's LDS words, which the first
     // barrier below completes (the global words are stored after it); rows of more words than
     // LDS holds go one word per wave at a time.
-        if (lds_bits)
+    if (lds_bits)
       for (int w = wave; w < nwords; w += W) sbits[sub][w][lane] = 0u;
     __syncthreads();
     if (lds_bits) {
@@ -492,9 +493,9 @@ void k_step_pack(StepPack p, EamArgs<S> a, int ngroups)
 //   1,024 atoms LJ float64 21 -> 9.8            1,048,576 atoms half list float32 292 -> 238
 //   8,192 atoms half list float64 24 -> 10.7    262,144 atoms LJ with ghost rows float32 169 -> 131
 //   131,072 atoms half list float64 53 -> 35    (about 2.5 TB/s of list and packed edges)
-// Measured beside it: two slots at a time 254 and 140 (the last two float32 cases), four waves 226
-// and 147, sixteen 319 and 153, the edges compacted in LDS and stored 16 bytes at a time 238 and
-// 131.
+// Measured beside it: two slots at a time 254 and 140 (the last two float32 cases), sixteen waves
+// 319 and 153, the edges compacted in LDS and stored 16 bytes at a time 238 and 131. Four waves take
+// 226 and 147: rows of 48 slots (the half list) gain less by them than rows of 78 lose.
 constexpr int kPackW = 8;      // waves per tile
 constexpr int kPackU = 4;      // slots of a row in flight per wave
 constexpr int kPackKeep = 128; // slots whose neighbours stay in LDS: 32 KB, four blocks per CU
@@ -681,7 +682,10 @@ void k_pack_rows(StepPack p, const Atom4<S> *__restrict__ atoms, int nlocal,
   }
 }
 
-// Rows of more than 256 slots, whose validity words LDS does not hold, take k_step_pack.
+// Lists with room for more than 256 slots, whose validity words LDS might not hold, take k_step_pack
+// at eight waves of dealt slots, also where their rows are shorter. LJ steps with such room, us, at
+// four waves of whole words before and now: 1,024 atoms float64 36.7 -> 29.7, 32,000 float32
+// 51.5 -> 45.4, 131,072 float64 124.7 -> 115.8 and float32 102.0 -> 95.2.
 template <typename S>
 static void launch_pack_rows(Handle &h, hipStream_t s, const StepPack &p, const EamArgs<S> &a,
                              int ntiles)

@@ -1015,11 +1015,16 @@ hipError_t launch_step_tiles(Handle &h, hipStream_t s, const double *x, const in
   };
   // Up to one tile per CU, each 64-row half of a tile takes a block of its own: both blocks stage
   // the tile's union, but twice the waves walk and write its rows and every CU still holds them all
-  // at once. us, whole tiles and halves (chosen starred):
-  //   8 tiles (1,008 atoms) 21.1, 15.3*   128 (16,384) 23.0, 17.4*   233 (29,716) 26.9, 23.2*
-  //   352 (45,056) 57.5*, 52.4            512 (65,536) 38.3*, 42.0   1,024 (131,072) 68.1*, 79.9
-  // (Halves of eight waves: 16.4, 18.7, 23.7 at the first three; of sixteen, one block per CU: 15.4,
-  // 17.8, 31.2.)
+  // at once. Past that they share CUs with other blocks and gain nothing, and from three tiles to
+  // two CUs the second staging costs more than the waves give. us, whole tiles and halves (chosen
+  // starred), of boxes whose tiles are all staged:
+  //   8 tiles (1,008 atoms) 21.1, 15.3*       264 (33,792) 35.9*, 35.8   432 (55,296) 37.1*, 42.1
+  //   128 (16,384)          23.0, 17.4*       320 (40,480) 35.7*, 35.4   512 (65,536) 39.1*, 43.4
+  //   256 (32,768)          30.0, 26.3*       384 (49,152) 35.6*, 36.2   1,024 (131,072) 68.1*, 79.9
+  // (Halves of eight waves: 16.4 and 18.7 at the first two; of sixteen, one block per CU: 15.4,
+  // 17.8.) A tile past the staging cap gathers its neighbours from memory and alone takes about 53
+  // (halves 49), so a box with one is timed by it: 272 tiles of 34 x 16 x 16 cells 53, 448 of
+  // 56 x 16 x 16 with 42 such tiles 72 (halves 87).
   if (t.ntiles <= (h.num_cus > 0 ? h.num_cus : 256))
     launch(std::integral_constant<int, 2 * kTileW>{}, std::integral_constant<int, 1>{});
   else

@@ -1701,8 +1701,12 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   // name and so its LDS counts (fewer claims in memory). Count and scatter together in us by waves
   // 2, 4, 8, 16, chosen starred; two at every size before:
   //   16 tiles (1,024 rows, plain)  65, 38, 26, 20*    1,024 tiles (65,536, plain) 81, 57*, 62, 88
-  //   128 tiles (8,192, half)       61, 37, 27*, 25    2,048 tiles (131,072, half) 74, 56*, 75, 98
-  //   500 tiles (32,000, plain)     76, 51, 45*, 53    4,000 tiles (256,000, half) 105*, 117, 134, 163
+  //   500 tiles (32,000, plain)     76, 51, 45*, 53    2,048 tiles (131,072, half) 74, 56*, 75, 98
+  //                                                    4,000 tiles (256,000, half) 105*, 117, 134, 163
+  // The line between sixteen and eight waves lies where they meet: both stages by events, 8 and 16,
+  //   64 tiles (4,096, plain)  42.6, 41.7*    192 tiles (12,288, half)  41.6*, 40.9
+  //   96 tiles (6,144, plain)  45.7*, 45.7    256 tiles (16,384, plain) 50.7*, 53.8
+  //   128 tiles (8,192, half)  40.2*, 38.8    400 tiles (25,600, half)  45.8*, 47.6
   const int cus = h.num_cus > 0 ? h.num_cus : 256, tiles = (L.rows + kWave - 1) / kWave;
   auto bins = [&](auto scatter, auto *tmp) {
     using E = std::remove_pointer_t<decltype(tmp)>;
