@@ -57,7 +57,7 @@ void free_all(Handle &h)
                   h.d_tile_off,  h.d_bits,      h.d_fp,          h.d_rho,       h.d_partials,
                   h.d_result,    h.d_ghost_owner, h.d_ghost_off, h.d_ghost_list, h.d_done,
                   h.d_deg,       h.d_inc_loc,   h.d_inc_part,    h.d_inc_tmp,   h.d_inc,
-                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,      h.d_inc_bit,
+                  h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,      h.d_inc_bit,   h.d_row_of,
                   h.d_matrix,    h.d_num_neighbors, h.d_identity, h.d_inc_len,
                   h.tl.keys,     h.tl.keys_sorted, h.tl.rows_in, h.tl.order,  h.tl.sort_tmp,
                   h.tl.atom,     h.tl.nn,       h.tl.uni,        h.tl.ucount,   h.tl.lid,
@@ -83,13 +83,20 @@ void mark_mirrored(Handle &h)
   ++h.mirror_expected;
 }
 
+// A validity-bit address holds its word in 27 bits, an entry on its way into the incidence lists its
+// slot in 26.
+bool slots_addressable(const Handle &h, int maxneighs)
+{
+  const long bit_words = static_cast<long>((maxneighs + 31L) / 32) * h.contract.max_atoms;
+  return bit_words < (1L << 27) && maxneighs <= (1 << 26);
+}
+
 // Two-sided incidence lists come from the list slots unless the pack's filter depends on the
-// positions (unique boundary) or duplicates edges, or a validity-bit address would not fit in
-// 27 bits.
+// positions (unique boundary) or duplicates edges, or a slot could not be addressed.
 bool incidence_from_list(const Handle &h)
 {
-  const long bit_words = static_cast<long>((h.list_maxneighs + 31) / 32) * h.contract.max_atoms;
-  return h.list_neighbors && !h.list_unique && !h.list_duplicate && bit_words < (1L << 27);
+  return h.list_neighbors && !h.list_unique && !h.list_duplicate &&
+         slots_addressable(h, h.list_maxneighs);
 }
 
 int ensure_bits(Handle &h, int maxneighs)
@@ -129,6 +136,8 @@ int ensure_incidence(Handle &h, long entries = 0)
     if ((e = get(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
     if ((e = get(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
     if ((e = get(&h.d_bins, lk::bin_words(A))) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bins)");
+    if (h.scalar_bytes() == 4 && h.list_bits_filter)
+      if ((e = get(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");
     if ((e = get_scalars(&h.d_rho_part)) != hipSuccess) return hip_fail(h, e, "hipMalloc(rho partials)");
     if ((e = get_scalars(&h.d_epair)) != hipSuccess) return hip_fail(h, e, "hipMalloc(pair energy)");
     if ((e = dalloc(&h.d_deg, A + 2)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence counts)");
@@ -153,10 +162,11 @@ int ensure_incidence(Handle &h, long entries = 0)
     h.d_inc = nullptr;
     h.d_inc_bit = nullptr;
     h.inc_cap = 0;
-    const long words = h.contract.max_atoms <= lk::kBinAtoms32 ? need : need + (need + 1) / 2;
+    const bool bits = h.scalar_bytes() == 4 && h.list_bits_filter;
+    const long words = bits || h.contract.max_atoms > lk::kBinAtoms32 ? need + (need + 1) / 2 : need;
     if ((e = dalloc(&h.d_inc_tmp, words)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence staging)");
     if ((e = dalloc(&h.d_inc, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lists)");
-    if (h.scalar_bytes() == 4 && h.list_bits_filter)
+    if (bits)
       if ((e = dalloc(&h.d_inc_bit, need)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bits)");
     h.inc_cap = need;
     h.inc_key = Handle::IncKey{};  // rebuild
@@ -821,8 +831,7 @@ int lk_pack_compute(lk_handle *w, void *stream, const double *x, const int *type
     long rows = static_cast<long>(inum) + (multi_hop ? gnum : 0);
     if (rows > c.max_atoms) rows = c.max_atoms;
     const int mnb = maxneighs > 1 ? maxneighs : 1;
-    const long bit_words = static_cast<long>((mnb + 31) / 32) * c.max_atoms;
-    if (!(half_edges && full_list) && bit_words < (1L << 27) && inum >= 0 && gnum >= 0 &&
+    if (!(half_edges && full_list) && slots_addressable(h, mnb) && inum >= 0 && gnum >= 0 &&
         nlocal >= 0 && nghost >= 0 && nall >= 0 && f) {
       if (static_cast<long>(nlocal) + nghost > c.max_atoms)
         return fail(h, LK_ERR_CAPACITY, "LAMMPS-JAX atom capacity exceeded");

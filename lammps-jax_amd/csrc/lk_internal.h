@@ -146,7 +146,7 @@ struct Handle {
   int *d_inc_loc = nullptr;     // [max_atoms + 1] offsets within each scan chunk
   int *d_inc_part = nullptr;    // [chunks] chunk offsets
   uint32_t *d_inc_tmp = nullptr;  // entries on their way into d_inc: [inc_cap] words, half as many
-                                  // again past kBinAtoms32 atoms
+                                  // again where they may take 64 bits (float32 and large capacities)
   int *d_inc = nullptr;         // [inc_cap] other atom | side << 31: an edge-built list's entries
                                 // in edge order; a list-built one's out-entries in slot order, then
                                 // its in-entries by row atom
@@ -170,6 +170,7 @@ struct Handle {
   // float32: each list-built entry's place among the validity bits, written for sweeps that follow
   // a pack called on its own (inc_bits: those of the lists that stand)
   uint32_t *d_inc_bit = nullptr;  // [inc_cap]
+  int *d_row_of = nullptr;        // [max_atoms] list row of each atom that is one, for their build
   bool inc_bits = false;
   // the neighbour list of the last lk_pack_edges: the two-sided incidence lists are built from
   // its slots once per list (lk_set_list_epoch) and filtered each step by the pack's bits

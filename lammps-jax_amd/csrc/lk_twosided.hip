@@ -253,12 +253,17 @@ struct ListArgs {
   int max_atoms;
   int half_filter;
   int *out_n;   // list slots of each atom's row (0: the atom is no row)
+  int *row_of;  // list row of each atom that is one; null without inc_bit
   int *loc;     // first entry of each atom
   int *part;    // zero (loc holds whole offsets)
   int *len;     // entries of each atom
   int *inc;
+  uint32_t *inc_bit;  // each entry's place among the validity bits, rows of words `bit_pitch` apart;
+                      // null: not wanted
+  int bit_pitch;
   uint32_t *claim;  // the sorted path's marks where LDS does not hold them, a word per in-entry
   int fold;         // the plain scheme's fold
+  int slots;        // the entries carry their slots
   BinLayout layout;
   int *longest;  // lists with room for longer rows than 64-atom bins take: the longest row, which
                  // the layout then goes by; else null
@@ -279,6 +284,13 @@ __device__ __forceinline__ bool list_neighbor(const ListArgs &L, int i, int jj, 
   j = L.neighbors[static_cast<long>(jj) * L.stride + i] & kNeighMask;
   if (j >= L.max_atoms) return false;
   return !(L.half_filter && j < i);
+}
+
+// The place of slot jj of list row ii among the validity bits: word (jj >> 5) * pitch + ii, bit jj & 31.
+__device__ __forceinline__ uint32_t slot_bit(const ListArgs &L, int ii, int jj)
+{
+  return ((static_cast<uint32_t>(jj >> 5) * static_cast<uint32_t>(L.bit_pitch) +
+           static_cast<uint32_t>(ii)) << 5) | static_cast<uint32_t>(jj & 31);
 }
 
 // An in-entry (row i names atom a) whose reverse slot is one of a's out-entries (a's row names
@@ -309,21 +321,54 @@ constexpr int kBinWaves = 16;            // waves of a counting block: kBinWaves
 constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
 constexpr int kBinProbes = 8;
 
-// An entry on its way: the atom's place in its bin above the row atom. 32 bits hold atoms below
-// 2^26 - 1.
+// An entry on its way: the atom's place in its bin above the row atom, in 32 bits where atoms stay
+// below 2^26 - 1; in 64 past that, and where the lists keep their slots' validity bit addresses: the
+// slot is then below the row atom.
 template <typename E>
-constexpr int kBinShift = sizeof(E) == 4 ? 26 : 32;
+struct Entry;
+template <>
+struct Entry<uint32_t> {
+  static constexpr bool kSlot = false;
+  static __device__ __forceinline__ uint32_t make(int place, int row_atom, int)
+  {
+    return (static_cast<uint32_t>(place) << 26) | static_cast<uint32_t>(row_atom);
+  }
+  static __device__ __forceinline__ uint32_t who(uint32_t v) { return v; }  // without the slot
+  static __device__ __forceinline__ int place(uint32_t v) { return static_cast<int>(v >> 26); }
+  static __device__ __forceinline__ uint32_t row_atom(uint32_t v) { return v & ((1u << 26) - 1); }
+  static __device__ __forceinline__ int slot(uint32_t) { return 0; }
+};
+template <>
+struct Entry<uint64_t> {
+  static constexpr bool kSlot = true;
+  static __device__ __forceinline__ uint64_t make(int place, int row_atom, int slot)
+  {
+    return (static_cast<uint64_t>(place) << 56) | (static_cast<uint64_t>(row_atom) << 26) |
+           static_cast<uint64_t>(slot);
+  }
+  static __device__ __forceinline__ uint64_t who(uint64_t v) { return v >> 26; }
+  static __device__ __forceinline__ int place(uint64_t v) { return static_cast<int>(v >> 56); }
+  static __device__ __forceinline__ uint32_t row_atom(uint64_t v)
+  {
+    return static_cast<uint32_t>(v >> 26) & ((1u << 30) - 1);
+  }
+  static __device__ __forceinline__ int slot(uint64_t v)
+  {
+    return static_cast<int>(v & ((1u << 26) - 1));
+  }
+};
 
 // Atoms per bin: 64, or fewer where the out-entries of that many rows and their in-entries (with
 // a fold, hash tables four fifths full at the longest row's length) would take more than kBinPool.
-// Rows past 1,763 slots (1,981 without a fold) keep bins of four atoms and sort.
-__host__ __device__ inline BinLayout bin_layout(long longest, bool fold)
+// Rows past 1,760 slots (1,980 without a fold) keep bins of four atoms and sort. Entries with slots
+// take 16 bits more each (rows past 1,376 and 1,584).
+__host__ __device__ inline BinLayout bin_layout(long longest, bool fold, bool slots)
 {
   const long per = fold ? (longest * 5 / 4 + 7) / 4 * 4 : (longest + 7) / 4 * 4;
-  const long pitch = longest | 1;
+  const long pitch = longest | 1, atom = 4 * (per + pitch) + (slots ? 2 * per : 0);
   BinLayout y{kBinLog, 0, 0};
-  while (y.bin_log > kBinMinLog && (4 * (per + pitch)) << y.bin_log > kBinPool) --y.bin_log;
-  if ((4 * (per + pitch)) << y.bin_log <= kBinPool) {
+  while (y.bin_log > kBinMinLog && atom << y.bin_log > kBinPool) --y.bin_log;
+  if (atom << y.bin_log <= kBinPool) {
     y.per_atom = static_cast<int>(per);
     y.pitch = static_cast<int>(pitch);
   }
@@ -336,7 +381,7 @@ __host__ __device__ inline BinLayout bin_layout(long longest, bool fold)
 // 700 and 6,390 at 1,700; by the rows it takes 164 at each (153 at room for 80).
 __device__ __forceinline__ BinLayout bin_layout_of(const ListArgs &L)
 {
-  return L.longest ? bin_layout(*L.longest, L.fold != 0) : L.layout;
+  return L.longest ? bin_layout(*L.longest, L.fold != 0, L.slots != 0) : L.layout;
 }
 
 __device__ __forceinline__ int bin_count(const ListArgs &L, const BinLayout &y)
@@ -411,6 +456,7 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   };
   if (!SCATTER && wq == 0 && i >= 0) {
     L.out_n[i] = nn;
+    if (L.row_of) L.row_of[i] = ii;
     const int q = slot_of(i >> bin_log);
     atomicAdd(q >= 0 ? &aux[q] : &B.out[i >> bin_log], nn);
   }
@@ -436,11 +482,11 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
         const uint64_t upto = (2ull << lane) - 1ull;  // lanes up to this one
         const uint64_t next = heads & ~upto;
         const int n = (next ? __builtin_ctzll(next) : kWave) - lane;  // a head's run
-        use(j, b, head, n, 63 - __builtin_clzll(heads & upto));
+        use(j, j0 + W * u, b, head, n, 63 - __builtin_clzll(heads & upto));
       }
     }
   };
-  walk([&](int, int b, bool head, int n, int) {
+  walk([&](int, int, int b, bool head, int n, int) {
     if (!head || b < 0) return;
     const int q = slot_of(b);
     if (q >= 0)
@@ -462,7 +508,7 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
   }
   if constexpr (SCATTER) {
     __syncthreads();
-    walk([&](int j, int b, bool head, int n, int first) {
+    walk([&](int j, int jj, int b, bool head, int n, int first) {
       int at = 0;
       if (head && b >= 0) {
         const int q = slot_of(b);
@@ -470,7 +516,7 @@ void k_inc_bins(ListArgs L, Bins B, E *__restrict__ tmp)
       }
       at = __shfl(at, first, kWave) + lane - first;
       if (b >= 0)
-        tmp[at] = (static_cast<E>(j & ((1 << bin_log) - 1)) << kBinShift<E>) | static_cast<E>(i);
+        tmp[at] = Entry<E>::make(j & ((1 << bin_log) - 1), i, jj);
     });
   }
 }
@@ -551,10 +597,11 @@ __device__ __forceinline__ int rank_of(const uint4 *v4, int n4, uint32_t v, int 
   return rank;
 }
 
-// One wave stores the `c` values of slots[0, n) below 2^31 (`n` a multiple of four) in ascending
-// order, the side bit set. Distinct values have the ranks 0 .. c - 1, which sum to c (c - 1) / 2;
-// any other sum means equal ones, and the ranks are taken again with ties broken.
-__device__ __forceinline__ void store_ranked(const uint32_t *slots, int n, int c, int *out)
+// One wave gives use(rank, value, index) the `c` values of slots[0, n) below 2^31 (`n` a multiple of
+// four) with their places in ascending order. Distinct values have the ranks 0 .. c - 1, which sum to
+// c (c - 1) / 2; any other sum means equal ones, and the ranks are taken again with ties broken.
+template <class Use>
+__device__ __forceinline__ void store_ranked(const uint32_t *slots, int n, int c, Use &&use)
 {
   const uint4 *v4 = reinterpret_cast<const uint4 *>(slots);
   const int lane = threadIdx.x & (kWave - 1);
@@ -563,14 +610,14 @@ __device__ __forceinline__ void store_ranked(const uint32_t *slots, int n, int c
     const uint32_t v = slots[q];
     if (v >> 31) continue;
     const int r = rank_of<false>(v4, n / 4, v, q);
-    out[r] = static_cast<int>(v | (1u << 31));
+    use(r, v, q);
     sum += r;
   }
   if (wave_sum(sum) == c * (c - 1) / 2) return;
   for (int q = lane; q < n; q += kWave) {
     const uint32_t v = slots[q];
     if (v >> 31) continue;
-    out[rank_of<true>(v4, n / 4, v, q)] = static_cast<int>(v | (1u << 31));
+    use(rank_of<true>(v4, n / 4, v, q), v, q);
   }
 }
 
@@ -637,7 +684,7 @@ template <typename E, bool FOLD>
 __global__ __launch_bounds__(kListThreads) LK_EIGHT_WAVES
 void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
 {
-  extern __shared__ __align__(16) uint32_t pool[];  // [atoms][per_atom], then [atoms][pitch]
+  extern __shared__ __align__(16) uint32_t pool[];  // [atoms][per_atom], [atoms][pitch], slots
   __shared__ int nin[kBinAtoms], nout[kBinAtoms], rown[kBinAtoms];
   __shared__ int start[kBinAtoms], seg[kBinAtoms], next[kBinAtoms];
   __shared__ int spill;
@@ -650,10 +697,10 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
   const int e0 = B.off[blockIdx.x], n = B.off[blockIdx.x + 1] - e0;
   const int slots = na * per_atom;
   uint32_t *outs = pool + slots;
-  auto atom_of = [](E v) { return static_cast<int>(v >> kBinShift<E>); };
-  auto row_atom = [](E v) {
-    return static_cast<uint32_t>(v & ((static_cast<E>(1) << kBinShift<E>) - 1));
-  };
+  // the in-entries' slots, which 16 bits hold: longer rows than these sort
+  uint16_t *in_slot = reinterpret_cast<uint16_t *>(outs + na * pitch);
+  auto atom_of = [](E v) { return Entry<E>::place(v); };
+  auto row_atom = [](E v) { return Entry<E>::row_atom(v); };
   if (tid < kBinAtoms) {
     nin[tid] = 0;
     nout[tid] = 0;
@@ -699,6 +746,8 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
         bool in = false;
         for (int probe = 0; probe < per_atom && !in; ++probe) {
           in = atomicCAS(&keys[h], kIncNone, row_atom(v)) == kIncNone;
+          if constexpr (Entry<E>::kSlot)
+            if (in) in_slot[atom_of(v) * per_atom + h] = static_cast<uint16_t>(Entry<E>::slot(v));
           if (++h == static_cast<uint32_t>(per_atom)) h = 0;
         }
         if (!in) spill = 1;
@@ -764,22 +813,36 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
       if constexpr (!FOLD) {
         for (int e = tid; e < n; e += kListThreads) {
           const E v = tmp[e0 + e];
-          const int d = atom_of(v);
-          pool[seg[d] + atomicAdd(&next[d], 1)] = row_atom(v);
+          const int d = atom_of(v), at = seg[d] + atomicAdd(&next[d], 1);
+          pool[at] = row_atom(v);
+          if constexpr (Entry<E>::kSlot) in_slot[at] = static_cast<uint16_t>(Entry<E>::slot(v));
         }
         __syncthreads();
       }
       for (int d = wave; d < na; d += kWaves) {
-        int *to = L.inc + start[d];
+        int to = start[d];
+        int ii = 0;
+        if constexpr (Entry<E>::kSlot)
+          if (L.inc_bit && rown[d] > 0) ii = L.row_of[a0 + d];
         for (int k = 0; k < rown[d]; k += kWave) {
           const uint32_t v = k + lane < rown[d] ? outs[d * pitch + k + lane] : kIncNone;
           const uint64_t M = wave_ballot(v != kIncNone);
-          if (v != kIncNone) to[lanes_below(M)] = static_cast<int>(v);
+          if (v != kIncNone) {
+            L.inc[to + lanes_below(M)] = static_cast<int>(v);
+            if constexpr (Entry<E>::kSlot)
+              if (L.inc_bit) L.inc_bit[to + lanes_below(M)] = slot_bit(L, ii, k + lane);
+          }
           to += __popcll(M);
         }
+        const int in0 = FOLD ? d * per_atom : seg[d];
         if (nin[d] > 0)
-          store_ranked(FOLD ? pool + d * per_atom : pool + seg[d],
-                       FOLD ? per_atom : (nin[d] + 3) & ~3, nin[d], to);
+          store_ranked(pool + in0, FOLD ? per_atom : (nin[d] + 3) & ~3, nin[d],
+                       [&](int r, uint32_t v, int q) {
+                         L.inc[to + r] = static_cast<int>(v | (1u << 31));
+                         if constexpr (Entry<E>::kSlot)
+                           if (L.inc_bit)
+                             L.inc_bit[to + r] = slot_bit(L, L.row_of[v], in_slot[in0 + q]);
+                       });
       }
       return;
     }
@@ -793,12 +856,13 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
   const int strips = na < kWaves ? kWaves / na : 1;  // of an atom
   auto sorted_lists = [&](const E *T, uint32_t *claims, bool in_lds) {
     for (int d = tid; d <= na; d += kListThreads)
-      first[d] = d < na ? lower_bound(T, n, static_cast<E>(d) << kBinShift<E>) : n;
+      first[d] = d < na ? lower_bound(T, n, Entry<E>::make(d, 0, 0)) : n;
+    auto same = [](E u, E v) { return Entry<E>::who(u) == Entry<E>::who(v); };
     // The place of the in-entry from row j to atom d, the first of equal ones, or -1.
     auto find = [&](int d, int j) -> int {
-      const E key = (static_cast<E>(d) << kBinShift<E>) | static_cast<E>(j);
+      const E key = Entry<E>::make(d, j, 0);
       const int at = lower_bound(T, n, key);
-      return at < n && T[at] == key ? at : -1;
+      return at < n && same(T[at], key) ? at : -1;
     };
     // A run's first entry: its row atom is named by a slot of the atom's own row, and by another.
     const int marks = (n + 31) >> 5;
@@ -837,11 +901,11 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
       const int at = find(d, j);
       if (at < 0 || !marked(again, at)) return at >= 0;
       const int mth = at + naming(d, jj, j);
-      return mth < n && T[mth] == T[at];
+      return mth < n && same(T[mth], T[at]);
     };
     auto folded = [&](int d, int e) -> bool {
       int at = e;
-      while (at > 0 && T[at - 1] == T[e]) --at;
+      while (at > 0 && same(T[at - 1], T[e])) --at;
       if (at == e || !marked(again, at)) return at == e && marked(named, at);
       return e - at < naming(d, rown[d], static_cast<int>(row_atom(T[e])));
     };
@@ -899,12 +963,18 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
     place();
     walk(
         [&](int u, int d, int jj, int j, int rank) {
-          L.inc[start[d] + strip_out[u] + rank] = static_cast<int>(
-              static_cast<uint32_t>(j) | (FOLD && paired(d, jj, j) ? kIncPaired : 0u));
+          const int at = start[d] + strip_out[u] + rank;
+          L.inc[at] = static_cast<int>(static_cast<uint32_t>(j) |
+                                       (FOLD && paired(d, jj, j) ? kIncPaired : 0u));
+          if constexpr (Entry<E>::kSlot)
+            if (L.inc_bit) L.inc_bit[at] = slot_bit(L, L.row_of[a0 + d], jj);
         },
         [&](int u, int d, int e, int rank) {
-          L.inc[start[d] + nout[d] + strip_in[u] + rank] =
-              static_cast<int>(row_atom(T[e]) | (1u << 31));
+          const int at = start[d] + nout[d] + strip_in[u] + rank;
+          L.inc[at] = static_cast<int>(row_atom(T[e]) | (1u << 31));
+          if constexpr (Entry<E>::kSlot)
+            if (L.inc_bit)
+              L.inc_bit[at] = slot_bit(L, L.row_of[row_atom(T[e])], Entry<E>::slot(T[e]));
         },
         [](int, int, int) {});
   };
@@ -924,50 +994,6 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
       sorted_lists(tmp + e0, head, true);
     else
       sorted_lists(tmp + e0, L.claim + e0, false);
-  }
-}
-
-// The place of each list entry's slot among the pack's validity bits (word (jj >> 5) * pitch + ii, bit
-// jj & 31, the words of a row `pitch` apart), for float32 sweeps after a pack called on its own:
-// one block per 64-row tile, the waves sharing its slots out in ranges. An out-entry's place follows
-// from the kept slots before it, an in-entry is found by bisection in the list of the atom its slot
-// names (out-entries come first, without the side bit, so the whole list is in order against the
-// key); the folded ones are not there, and equal ones stand for equal slots. Once per list and only
-// for such calls (46 us at 62,500 atoms of a half list). A search of the sender's row in the sweeps,
-// for every entry near the cutoff, read the engine's list on every step and, with a neighbour shell
-// on the cutoff, took 46.6 us of that box's density sweep and 56.8 of its force sweep, now 16.0 and
-// 29.6.
-constexpr int kBitWaves = 16;
-
-__global__ __launch_bounds__(kBitWaves *kWave) LK_EIGHT_WAVES
-void k_inc_bits(ListArgs L, int pitch, uint32_t *__restrict__ inc_bit)
-{
-  __shared__ int kept[kBitWaves][kWave];
-  const int wave = wave_in_block(), lane = threadIdx.x & (kWave - 1);
-  const int ii = blockIdx.x * kWave + lane;
-  int nn = 0, i = -1;
-  if (ii < L.rows) i = list_row(L, ii, nn);
-  const int nmax = wave_max_int(nn), per = (nmax + kBitWaves - 1) / kBitWaves;
-  const int j0 = min(wave * per, nn), j1 = min(j0 + per, nn);
-  int c = 0;
-  for (int jj = j0; jj < j1; ++jj) {
-    int j;
-    c += list_neighbor(L, i, jj, j) ? 1 : 0;
-  }
-  kept[wave][lane] = c;
-  __syncthreads();
-  int at = i >= 0 ? L.loc[i] : 0;
-  for (int w = 0; w < wave; ++w) at += kept[w][lane];
-  for (int jj = j0; jj < j1; ++jj) {
-    int j;
-    if (!list_neighbor(L, i, jj, j)) continue;
-    const uint32_t bit = ((static_cast<uint32_t>(jj >> 5) * static_cast<uint32_t>(pitch) +
-                           static_cast<uint32_t>(ii)) << 5) | static_cast<uint32_t>(jj & 31);
-    inc_bit[at++] = bit;
-    const uint32_t *list = reinterpret_cast<const uint32_t *>(L.inc) + L.loc[j];
-    const uint32_t key = static_cast<uint32_t>(i) | (1u << 31);
-    const int n = L.len[j];
-    for (int q = lower_bound(list, n, key); q < n && list[q] == key; ++q) inc_bit[L.loc[j] + q] = bit;
   }
 }
 
@@ -995,7 +1021,7 @@ struct TwoSided {
   const int *ghost_list;
   int nblk;             // 64-atom partial tiles over nall
   const uint32_t *bits;     // kFromBits: the pack's validity bits
-  const uint32_t *inc_bit;  // kFromBits: each entry's place in them (k_inc_bits)
+  const uint32_t *inc_bit;  // kFromBits: each entry's place in them
   double cutsq_pack;        // the pack's filter: rsq <= cutsq in float64 (cpp:91)
   float cutsq_lo, cutsq_hi; // cutsq_pack rounded down and up to float
   const int *ghost_flag;    // 1 when a packed edge starts on a ghost row (the pack's flag)
@@ -1663,7 +1689,7 @@ static hipError_t build_incidence(Handle &h, hipStream_t s, int nall)
   return hipGetLastError();
 }
 
-static ListArgs list_args(Handle &h, bool fold)
+static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold, bool bits)
 {
   ListArgs L{};
   L.ilist = h.list_ilist;
@@ -1680,14 +1706,12 @@ static ListArgs list_args(Handle &h, bool fold)
   L.len = h.d_inc_len;
   L.inc = h.d_inc;
   L.fold = fold ? 1 : 0;
-  L.layout = bin_layout(L.maxneighs, fold);
-  return L;
-}
-
-static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
-{
-  ListArgs L = list_args(h, fold);
   const int atoms = L.max_atoms;
+  L.slots = bits || atoms > kBinAtoms32 ? 1 : 0;
+  L.layout = bin_layout(L.maxneighs, fold, L.slots != 0);
+  L.inc_bit = bits ? h.d_inc_bit : nullptr;
+  L.row_of = bits ? h.d_row_of : nullptr;
+  L.bit_pitch = h.contract.max_atoms;
   Bins B;
   B.cap = (atoms + (1 << L.layout.bin_log) - 1) >> L.layout.bin_log;
   B.next = h.d_bins;
@@ -1697,7 +1721,9 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
   const bool measure = L.layout.bin_log < kBinLog;
   L.longest = measure ? B.loff + B.cap : nullptr;
   const size_t lds = measure ? kBinPool
-                             : static_cast<size_t>(4 * (L.layout.per_atom + L.layout.pitch)) << kBinLog;
+                             : static_cast<size_t>(4 * (L.layout.per_atom + L.layout.pitch) +
+                                                   (L.slots ? 2 * L.layout.per_atom : 0))
+                                   << kBinLog;
   // Waves per 64-row tile of the counting blocks: many where the tiles are few, so that the blocks
   // reach the CUs; two past eight tiles per CU, where a block's eight tiles share the bins they
   // name and so its LDS counts (fewer claims in memory). Count and scatter together in us by waves
@@ -1754,8 +1780,8 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold)
                          tmp, static_cast<int>(lds / 4));
   };
   // d_inc_tmp holds an entry and a word of marks per list slot (ensure_incidence)
-  L.claim = h.d_inc_tmp + static_cast<long>(L.rows) * L.maxneighs * (atoms <= kBinAtoms32 ? 1 : 2);
-  if (atoms <= kBinAtoms32)
+  L.claim = h.d_inc_tmp + static_cast<long>(L.rows) * L.maxneighs * (L.slots ? 2 : 1);
+  if (!L.slots)
     finish(h.d_inc_tmp);
   else
     finish(reinterpret_cast<uint64_t *>(h.d_inc_tmp));
@@ -1777,39 +1803,29 @@ static Handle::IncKey list_key(const Handle &h, bool fold)
 }
 
 // The incidence lists of the neighbour list, built once per list: by the engine's epoch (or every
-// step when it gives none) and the list's shape. A build that failed leaves no lists to reuse.
-static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold)
+// step when it gives none) and the list's shape; `bits`: with the entries' validity bit addresses,
+// for sweeps that read them. A build that failed leaves no lists to reuse.
+static hipError_t lists_of_list(Handle &h, hipStream_t s, bool fold, bool bits)
 {
   const Handle::IncKey key = list_key(h, fold);
-  if (h.list_epoch >= 0 && key == h.inc_key) return hipSuccess;
+  if (h.list_epoch >= 0 && key == h.inc_key && (!bits || h.inc_bits)) return hipSuccess;
   h.inc_key = Handle::IncKey{};
-  h.inc_bits = false;
-  const hipError_t e = build_incidence_from_list(h, s, fold);
-  if (e == hipSuccess) h.inc_key = key;
+  const hipError_t e = build_incidence_from_list(h, s, fold, bits);
+  if (e == hipSuccess) {
+    h.inc_key = key;
+    h.inc_bits = bits;
+  }
   return e;
 }
 
-// The places of the lists' entries among the validity bits, for the sweeps that read them.
-static hipError_t bits_of_list(Handle &h, hipStream_t s)
-{
-  if (h.inc_bits || !h.d_inc_bit) return hipSuccess;
-  const ListArgs L = list_args(h, h.inc_key.fold != 0);
-  const int tiles = (L.rows + kWave - 1) / kWave;
-  StageTimer timer(h, s, "inc_bits");
-  if (tiles > 0)
-    hipLaunchKernelGGL(k_inc_bits, dim3(tiles), dim3(kBitWaves * kWave), 0, s, L,
-                       h.contract.max_atoms, h.d_inc_bit);
-  const hipError_t e = hipGetLastError();
-  h.inc_bits = e == hipSuccess;
-  return e;
-}
-
-// A pack called on its own over the list that the incidence lists already stand for: what its sweeps
-// will need of the list is read here, so that they read no list on a step that rebuilds none.
+// A pack called on its own over the list that incidence lists without bit addresses stand for (a fused
+// step built them): its sweeps will want the addresses, and the list is there to read now.
 hipError_t launch_list_bits(Handle &h, hipStream_t s)
 {
-  if (h.list_epoch < 0 || !(list_key(h, h.inc_key.fold != 0) == h.inc_key)) return hipSuccess;
-  return bits_of_list(h, s);
+  const bool fold = h.inc_key.fold != 0;
+  if (h.list_epoch < 0 || h.inc_bits || !h.d_inc_bit || !(list_key(h, fold) == h.inc_key))
+    return hipSuccess;
+  return lists_of_list(h, s, fold, true);
 }
 
 // The incidence lists of the packed edges, built every step.
@@ -1825,6 +1841,13 @@ static int sweep_filter(const Handle &h, bool from_list, const FusedPack &pack)
 {
   if (!from_list || !h.list_bits_filter) return kAllKept;
   return pack.state ? kFromX : kFromBits;
+}
+
+// Whether sweeps over the list's entries after this pack read validity bits (float64 ones decide every
+// entry from its own r2).
+static bool reads_bits(const Handle &h, const FusedPack &pack)
+{
+  return h.d_inc_bit && sweep_filter(h, true, pack) == kFromBits;
 }
 
 // Calls f with `filter` as a constant. Float64 sweeps decide every entry from its own r2, so one
@@ -2299,8 +2322,7 @@ hipError_t launch_edge_force(Handle &h, hipStream_t s, int nlocal, int nghost, i
                : lj_edge_force<float>(h, s, nlocal, nghost, flags, scale, f, x);
   hipError_t e = hipSuccess;
   if (from_list) {
-    e = lists_of_list(h, s, false);  // the edge-force sweeps walk whole lists
-    if (e == hipSuccess && sweep_filter(h, true, FusedPack{}) == kFromBits) e = bits_of_list(h, s);
+    e = lists_of_list(h, s, false, reads_bits(h, FusedPack{}));  // whole lists
   } else {
     e = lists_of_edges(h, s, nlocal + nghost);
   }
@@ -2317,8 +2339,7 @@ hipError_t launch_two_sided(Handle &h, hipStream_t s, int nlocal, int nghost, in
   if (phase == kPhaseForce) {
     // the incidence lists are the ones this step's density pass used
   } else if (from_list) {
-    e = lists_of_list(h, s, h.accum == LK_ACCUM_PLAIN);
-    if (e == hipSuccess && sweep_filter(h, true, pack) == kFromBits) e = bits_of_list(h, s);
+    e = lists_of_list(h, s, h.accum == LK_ACCUM_PLAIN, reads_bits(h, pack));
   } else {
     e = lists_of_edges(h, s, nlocal + nghost);
   }

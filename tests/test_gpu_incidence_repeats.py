@@ -2,7 +2,7 @@
 
 Each repeated slot is an edge of its own (the pack keeps every one), so the plain scheme's fold has
 to pair slots one to one whichever path builds the lists: hash tables in LDS, or a sort of the bin's
-entries (rows past 1,763 slots, bins that more entries name than LDS holds, rows that repeat an atom
+entries (rows past 1,760 slots, bins that more entries name than LDS holds, rows that repeat an atom
 whose own row names them back). Rows repeat some of their neighbours once or twice, some in both
 directions and some in one; in the longer cases a third of the rows is filled with atoms past the
 cutoff, many of them repeated too, up to the length under test, and `hubs` gives every row far atoms

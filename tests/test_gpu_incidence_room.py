@@ -1,7 +1,7 @@
 """The list-built incidence lists go by the rows of a list, not by the room it has for them.
 
 An engine's list may have room for far more slots than any row uses (it grows by the widest row ever
-seen). Past the room that bins of 64 atoms take (107 slots with the plain scheme's fold, 119
+seen). Past the room that bins of 64 atoms take (107 slots with the plain scheme's fold, 120
 without), the build measures the longest row first and sizes its bins by it: 64, 32, 16, 8 and 4
 atoms are reached here by rows given distinct atoms past the cutoff, each with tight room and with
 room for 2,500 slots. Against the oracle, and the same forces bit for bit at either room."""

@@ -6,7 +6,9 @@ and no longer: on later steps of the same list its arrays may change once lk_pac
 called, also where the lists were built by the fused step, which needs no bits. The engine here
 overwrites them (with other valid entries) between the pack and the model pass. A perturbed lattice
 cut at its second-shell distance, so that about half of that shell is kept and float32 decides none
-of it. Against the oracle, and each step with the first bit for bit."""
+of it: rows as the list has them, rows made longer by far atoms (bins of fewer atoms, and bins whose
+entries are sorted) and rows that name some of the shell twice. Against the oracle, and each step with
+the first bit for bit."""
 
 from __future__ import annotations
 
@@ -49,10 +51,38 @@ def _split(pj):
     return pj.h.step_result(st)
 
 
+def _longer(sysm, longest, twice):
+    """The list with every third row filled up to `longest` slots by atoms past the cutoff, ahead of
+    its own, and with `twice` half the rows naming one of their neighbours again."""
+    lst = dict(sysm.list)
+    stride, rows = lst["stride"], lst["maxneighs"]
+    old = np.asarray(lst["neighbors"]).reshape(rows, stride) & 0x3FFFFFFF
+    num = np.array(lst["numneigh"], copy=True)
+    nb = np.zeros((max(rows + 1, longest), stride), np.int32)
+    nb[:rows] = old
+    x = sysm.x[:sysm.nall]
+    rng = np.random.default_rng(9)
+    for n, i in enumerate(np.asarray(lst["ilist"])[:lst["inum"]]):
+        own = old[:num[i], i]
+        if twice and n % 2 and len(own):
+            own = np.insert(own, rng.integers(0, len(own) + 1), rng.choice(own))
+        far = np.flatnonzero(np.sum((x - x[i]) ** 2, axis=1) > (A + 0.1) ** 2)
+        add = np.resize(far, max(0, longest - len(own)) if n % 3 == 0 else 0)
+        num[i] = len(add) + len(own)
+        nb[:num[i], i] = np.concatenate([add, own])
+    lst.update(neighbors=np.ascontiguousarray(nb.reshape(-1)), numneigh=num, maxneighs=len(nb))
+    sysm.list = lst
+    return lst
+
+
 @pytest.mark.parametrize("first", ["fused", "split"])
-@pytest.mark.parametrize("scheme,cells", [("half", (5, 5, 5)), ("half", (9, 8, 8)),
-                                          ("plain", (5, 5, 5)), ("plain lj", (9, 8, 7))])
-def test_split_steps_on_a_standing_list(gpu, scheme, cells, first):
+@pytest.mark.parametrize("scheme,cells,longest,twice", [
+    ("half", (5, 5, 5), 0, False), ("half", (9, 8, 8), 0, False), ("plain", (5, 5, 5), 0, False),
+    ("plain lj", (9, 8, 7), 0, False), ("half", (5, 5, 5), 300, False),
+    ("plain", (4, 5, 5), 200, False), ("half", (5, 4, 5), 1700, False),
+    ("plain lj", (5, 5, 4), 1500, False), ("plain lj", (5, 5, 5), 0, True),
+    ("half", (5, 5, 5), 0, True), ("plain", (5, 4, 5), 1500, True)])
+def test_split_steps_on_a_standing_list(gpu, scheme, cells, longest, twice, first):
     half, lj = scheme == "half", scheme.endswith("lj")
     box = np.array(cells, float) * A
     rng = np.random.default_rng(5)
@@ -65,9 +95,12 @@ def test_split_steps_on_a_standing_list(gpu, scheme, cells, first):
         model = ("eam", systems.synthetic_alloy_tables(cutoff=A))
     sysm = systems.System(x, types, box, A + 1.0)
     lst = sysm.build_list(A + 1.0, kind=harness.LIST_HALF if half else harness.LIST_FULL)
+    if longest or twice:
+        lst = _longer(sysm, longest, twice)
     pj = PairJax(sysm, model, precision=4, accumulation=scheme.split()[0])
     nl, nall = sysm.nlocal, sysm.nall
-    print(f"split filter {scheme} cells={cells} first={first} nall={nall}", flush=True)
+    print(f"split filter {scheme} cells={cells} room={lst['maxneighs']} first={first} nall={nall}",
+          flush=True)
     pos, sp = O.pack_atoms(sysm.x, sysm.type, nall, pj.max_atoms, 4)
     s, r, m, count, _ = O.pack_neighbors(sysm.x, lst, max_atoms=pj.max_atoms,
                                          max_edges=pj.max_edges, nlocal=nl, cutoff=A)
