@@ -58,7 +58,7 @@ void free_all(Handle &h)
                   h.d_result,    h.d_ghost_owner, h.d_ghost_off, h.d_ghost_list, h.d_done,
                   h.d_deg,       h.d_inc_loc,   h.d_inc_part,    h.d_inc_tmp,   h.d_inc,
                   h.d_rho_part,  h.d_epair,     h.d_pack_state,  h.d_bins,      h.d_edge_f,      h.d_inc_bit,   h.d_row_of,
-                  h.d_matrix,    h.d_num_neighbors, h.d_identity, h.d_inc_len,
+                  h.d_matrix,    h.d_num_neighbors, h.d_identity, h.d_inc_span,
                   h.tl.keys,     h.tl.keys_sorted, h.tl.rows_in, h.tl.order,  h.tl.sort_tmp,
                   h.tl.atom,     h.tl.nn,       h.tl.uni,        h.tl.ucount,   h.tl.lid,
                   h.tl.box,      h.d_rowmark,   h.d_nonrow,      h.d_htab,      h.tl.ustat, h.d_dtab};
@@ -134,7 +134,7 @@ int ensure_incidence(Handle &h, long entries = 0)
     auto get_scalars = [&](void **p) { return *p ? hipSuccess : hipMalloc(p, A * h.scalar_bytes()); };
     if ((e = get(&h.d_inc_loc, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence offsets)");
     if ((e = get(&h.d_inc_part, chunks)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence chunks)");
-    if ((e = get(&h.d_inc_len, A + 1)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
+    if ((e = get(&h.d_inc_span, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence lengths)");
     if ((e = get(&h.d_bins, lk::bin_words(A))) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence bins)");
     if (h.scalar_bytes() == 4 && h.list_bits_filter)
       if ((e = get(&h.d_row_of, A)) != hipSuccess) return hip_fail(h, e, "hipMalloc(incidence rows)");

@@ -143,14 +143,16 @@ struct Handle {
   // incidence lists of the two-sided schemes (lk_twosided.hip), allocated on first use
   int *d_deg = nullptr;         // [max_atoms + 2] per-atom counts of the edge-built lists, slots of
                                 // each atom's row for the list-built ones
-  int *d_inc_loc = nullptr;     // [max_atoms + 1] offsets within each scan chunk
-  int *d_inc_part = nullptr;    // [chunks] chunk offsets
+  int *d_inc_loc = nullptr;     // [max_atoms + 1] edge-built: offsets within each scan chunk
+  int *d_inc_part = nullptr;    // [chunks] edge-built: chunk offsets
   uint32_t *d_inc_tmp = nullptr;  // entries on their way into d_inc: [inc_cap] words, half as many
                                   // again where they may take 64 bits (float32 and large capacities)
   int *d_inc = nullptr;         // [inc_cap] other atom | side << 31: an edge-built list's entries
                                 // in edge order; a list-built one's out-entries in slot order, then
                                 // its in-entries by row atom
-  int *d_inc_len = nullptr;     // [max_atoms + 1] entries of each atom in d_inc
+  int2 *d_inc_span = nullptr;   // [max_atoms] first entry and entries of each atom in d_inc, one load
+                                // of the sweeps (as three loads the float32 half scheme's matrix step
+                                // took 52.6 and 113.3 us at 32,000 and 131,072 atoms, now 51.0 and 108.6)
   void *d_rho_part = nullptr;   // [max_atoms] per-row density before the ghost fold
   void *d_epair = nullptr;      // [max_atoms] per-row pair energy
   const double *x_last = nullptr;  // engine positions of the last pack (f.r virial)

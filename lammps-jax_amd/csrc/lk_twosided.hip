@@ -62,7 +62,7 @@ struct IncArgs {
   int *part;  // [chunks] exclusive chunk offsets
   uint32_t *tmp;
   int *inc;
-  int *len;   // [nrows + 1] entries of each atom's list
+  int2 *span;  // [nrows] first entry and entries of each atom's list
 };
 
 __device__ __forceinline__ long live_edges(const StepResult *r, int max_edges)
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void k_inc_sort(IncArgs a, int nsort)
   if (atom >= nsort) return;  // whole wave
   const int b = inc_off(a.loc, a.part, atom);
   const int L = inc_off(a.loc, a.part, atom + 1) - b;
-  if (lane == 0) a.len[atom] = L;
+  if (lane == 0) a.span[atom] = make_int2(b, L);
   for (int c0 = 0; c0 < L; c0 += kWave) {
     const bool mine = c0 + lane < L;
     const uint32_t v = mine ? a.tmp[b + c0 + lane] : 0xFFFFFFFFu;
@@ -254,9 +254,7 @@ struct ListArgs {
   int half_filter;
   int *out_n;   // list slots of each atom's row (0: the atom is no row)
   int *row_of;  // list row of each atom that is one; null without inc_bit
-  int *loc;     // first entry of each atom
-  int *part;    // zero (loc holds whole offsets)
-  int *len;     // entries of each atom
+  int2 *span;   // first entry and entries of each atom
   int *inc;
   uint32_t *inc_bit;  // each entry's place among the validity bits, rows of words `bit_pitch` apart;
                       // null: not wanted
@@ -415,7 +413,6 @@ __global__ __launch_bounds__(256) void k_inc_clear(ListArgs L, Bins B)
     B.next[i] = 0;
     B.out[i] = 0;
   }
-  if (i < (L.max_atoms + kScanChunk) / kScanChunk) L.part[i] = 0;
 }
 
 // Count (SCATTER false: the in- and out-entries of each bin; also out_n) and scatter.
@@ -727,8 +724,7 @@ void k_inc_lists(ListArgs L, Bins B, E *__restrict__ tmp, int pool_words)
       seg[lane] = incl4 - c4;
       if (!FOLD && incl4 > slots) spill = 1;  // the half scheme's segments
       if (lane < na && a0 + lane < L.max_atoms) {
-        L.loc[a0 + lane] = start[lane];
-        L.len[a0 + lane] = c;
+        L.span[a0 + lane] = make_int2(start[lane], c);
       }
     }
     __syncthreads();
@@ -1007,10 +1003,8 @@ __device__ __forceinline__ T group_sum(T v)
 
 // Arguments of the two-sided sweeps besides the model block.
 struct TwoSided {
-  const int *loc;
-  const int *part;
+  const int2 *span;  // first entry and entries of each atom
   const int *inc;
-  const int *len;  // entries of each atom
   int nall;
   int nlocal;
   int nadd;             // rows that take the force add: nall with newton on, else nlocal
@@ -1189,8 +1183,8 @@ void k_eam_density_inc(EamArgs<S> m, TwoSided t, S *__restrict__ rho_part, S *__
       const Atom4<S> xa = m.atoms[a];
       const BandRow<S> br = band_row(t, xa, m.cutsq);
       const int za = clamp_species(static_cast<int>(xa.w), m.n_el);
-      const int b = inc_off(t.loc, t.part, a);
-      const int L = t.len[a];
+      const int2 span = t.span[a];
+      const int b = span.x, L = span.y;
       // Two entries per lane at a time (k and k + G): both entries load together, then both
       // records, so a pair of entries costs two memory round trips; a skipped or missing entry
       // gathers the row's own record.
@@ -1370,8 +1364,8 @@ __device__ __forceinline__ void eam_force_inc_rows(const EamArgs<S> &m, const Tw
       const BandRow<S> br = band_row(t, xa, m.cutsq);
       const int za = clamp_species(static_cast<int>(xa.w), m.n_el);
       const S fpa = m.fp[a];
-      const int b = inc_off(t.loc, t.part, a);
-      const int L = t.len[a];
+      const int2 span = t.span[a];
+      const int b = span.x, L = span.y;
       // The gathers of an entry: its neighbour's record and F' (the row's own when the entry
       // is skipped, so no branch surrounds a load).
       struct Gathered {
@@ -1579,8 +1573,8 @@ void k_lj_inc(LjModel<S> m, TwoSided t)
     if (a < t.nall) {
       const Atom4<S> xa = m.atoms[a];
       const BandRow<S> br = band_row(t, xa, m.cutsq);
-      const int b = inc_off(t.loc, t.part, a);
-      const int L = t.len[a];
+      const int2 span = t.span[a];
+      const int b = span.x, L = span.y;
       // counted ends of an entry: its sender's row, or both rows of a folded pair (the pair
       // force on a is the same from either directed edge)
       auto ends = [&](uint32_t v) -> int {
@@ -1659,7 +1653,7 @@ static hipError_t build_incidence(Handle &h, hipStream_t s, int nall)
   ia.part = h.d_inc_part;
   ia.tmp = h.d_inc_tmp;
   ia.inc = h.d_inc;
-  ia.len = h.d_inc_len;
+  ia.span = h.d_inc_span;
   const int egrid = grid_for(h, h.contract.max_edges, 256, 16);
   {
     StageTimer timer(h, s, "inc_count");
@@ -1701,9 +1695,7 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold,
   L.max_atoms = h.contract.max_atoms;
   L.half_filter = h.list_half_filter;
   L.out_n = h.d_deg;
-  L.loc = h.d_inc_loc;
-  L.part = h.d_inc_part;
-  L.len = h.d_inc_len;
+  L.span = h.d_inc_span;
   L.inc = h.d_inc;
   L.fold = fold ? 1 : 0;
   const int atoms = L.max_atoms;
@@ -1866,10 +1858,8 @@ static void with_filter(int filter, F &&f)
 static TwoSided two_sided_args(Handle &h, int nlocal, int nghost, const double *x)
 {
   TwoSided t;
-  t.loc = h.d_inc_loc;
-  t.part = h.d_inc_part;
+  t.span = h.d_inc_span;
   t.inc = h.d_inc;
-  t.len = h.d_inc_len;
   t.nall = nlocal + nghost;
   t.nlocal = nlocal;
   t.nadd = h.contract.newton_pair ? t.nall : nlocal;
