@@ -263,7 +263,7 @@ struct ListArgs {
   int fold;         // the plain scheme's fold
   int slots;        // the entries carry their slots
   BinLayout layout;
-  int *longest;  // lists with room for longer rows than 64-atom bins take: the longest row, which
+  int *longest;  // lists with room for longer rows than 32-atom bins take: the longest row, which
                  // the layout then goes by; else null
 };
 
@@ -314,6 +314,7 @@ constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 // of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
 constexpr int kBinLog = 6;
 constexpr int kBinAtoms = 1 << kBinLog;  // at most
+constexpr int kBinMeasureLog = 5;        // room for smaller bins than this: the rows are measured
 constexpr int kBinPool = 62 * 1024;      // LDS of a bin's lists (two blocks or more share a CU)
 constexpr int kBinWaves = 16;            // waves of a counting block: kBinWaves / W 64-row tiles
 constexpr int kBinTable = 2048;          // bins a block counts in LDS; others go to memory at once
@@ -374,9 +375,11 @@ __host__ __device__ inline BinLayout bin_layout(long longest, bool fold, bool sl
 }
 
 // An engine's list may have room for far more slots than its rows have, so where the room alone
-// would make the bins smaller the rows are measured on the device first. By the room, the step on a
-// new list of 32,000 LJ atoms with 80 slots a row (plain) took 245 us at room for 240 slots, 998 at
-// 700 and 6,390 at 1,700; by the rows it takes 164 at each (153 at room for 80).
+// would make the bins smaller than 32 atoms the rows are measured on the device first. By the room,
+// the step on a new list of 32,000 LJ atoms with 80 slots a row (plain) took 245 us at room for 240
+// slots, 998 at 700 and 6,390 at 1,700; by the rows it takes 164 at each (153 at room for 80). The
+// measuring takes 10 to 14 us: rows that do fill room for 108 to 218 slots would lose that for
+// nothing.
 __device__ __forceinline__ BinLayout bin_layout_of(const ListArgs &L)
 {
   return L.longest ? bin_layout(*L.longest, L.fold != 0, L.slots != 0) : L.layout;
@@ -1710,12 +1713,12 @@ static hipError_t build_incidence_from_list(Handle &h, hipStream_t s, bool fold,
   B.out = B.next + B.cap;
   B.off = B.out + B.cap;
   B.loff = B.off + B.cap + 1;
-  const bool measure = L.layout.bin_log < kBinLog;
+  const bool measure = L.layout.bin_log < kBinMeasureLog;
   L.longest = measure ? B.loff + B.cap : nullptr;
   const size_t lds = measure ? kBinPool
                              : static_cast<size_t>(4 * (L.layout.per_atom + L.layout.pitch) +
                                                    (L.slots ? 2 * L.layout.per_atom : 0))
-                                   << kBinLog;
+                                   << L.layout.bin_log;
   // Waves per 64-row tile of the counting blocks: many where the tiles are few, so that the blocks
   // reach the CUs; two past eight tiles per CU, where a block's eight tiles share the bins they
   // name and so its LDS counts (fewer claims in memory). Count and scatter together in us by waves
