@@ -311,7 +311,7 @@ constexpr uint32_t kIncNone = 0xFFFFFFFFu;
 // the same from run to run. The list is read four times, the entries written twice and read twice;
 // a radix sort of (atom, slot) pairs, the placing of out- and in-entries and the fold went over
 // the entries nine times: build of 256,000 atoms' half list (12.6 M entries) 566 -> 261 us,
-// of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 346 us.
+// of a 131,072-atom list with ghost rows (14 M entries, nearly all folded) 890 -> 295 us.
 constexpr int kBinLog = 6;
 constexpr int kBinAtoms = 1 << kBinLog;  // at most
 constexpr int kBinMeasureLog = 5;        // room for smaller bins than this: the rows are measured
