@@ -1,10 +1,12 @@
 """The list-built incidence lists of the two-sided schemes at the edges of their binned build.
 
 The build brings each bin's entries (the slots naming its atoms) together in LDS: 64 atoms to a bin,
-fewer the wider the list (`maxneighs` is padded here, as an engine's list may be), and a search in
-memory for rows past 1,700 slots or for bins that more entries name than LDS holds (every row given
-far atoms of one bin, which the cutoff drops again; in the plain scheme they have no reverse).
-Each is compared with the oracle, and a rebuild of the same list with the first build bit for bit."""
+fewer where the list's room asks for it; past 218 slots of room (`maxneighs` is padded here, as an
+engine's list may be) it measures the rows first and goes by the longest. Bins that more entries name
+than LDS holds sort them (every row given far atoms of one bin, which the cutoff drops again; in the
+plain scheme they have no reverse). Rows that are long themselves: test_gpu_incidence_room.py and
+test_gpu_incidence_repeats.py. Each is compared with the oracle, and a rebuild of the same list with
+the first build bit for bit."""
 
 from __future__ import annotations
 
